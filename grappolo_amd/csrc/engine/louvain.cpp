@@ -439,14 +439,29 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         color_nonempty[c] = size > 0;
         max_class = std::max(max_class, size);
     }
+    int nonempty = 0;
+    for (int c = 0; c < ncol; c++) nonempty += color_nonempty[c];
+    const i64 per_class = (nv + std::max(nonempty, 1) - 1) / std::max(nonempty, 1);
+    // graphs above the dense sweep's vertices: the whole-GPU persistent sweep
+    // (wide.hpp), plain form only.  Classes of more than kWideMaxPerColor
+    // vertices on average fill the GPU with per-color launches of the binned
+    // kernels.  Below 262,144 vertices it takes the place of those launches
+    // and of the hash form of the persistent sweep: a 250,007-vertex RMAT run
+    // went from 363 to 103 ms (its per-color launches took 13 ms per
+    // iteration, most of it one HBM-table launch per class), a 62,103-vertex
+    // coarse phase of 69 colors from 45.2 to 14.9 ms; dense phases (<= 15,360
+    // vertices) are no faster here as long as their classes are small.
+    const bool las_mode = las && !(las->mode == 2 && nv <= kDenseMaxNV) && las->mode != 0;
+    int wblocks = 0;
+    if (!las_mode && nv > kDenseMaxNV && nonempty > 0 && nv / nonempty <= kWideMaxPerColor && wide_enabled()) {
+        wblocks = wide_grid(g.nnz / nonempty);
+        if (tune_.wide_blocks > 0) wblocks = std::min(wblocks, tune_.wide_blocks);
+    }
     // coarse graphs (small, or many small color classes): one persistent
     // launch per iteration (all colors + modularity), grid sized to the color
     // classes: every extra workgroup only lengthens the barriers
     int pblocks = 0;
-    if (nv <= kPersistMaxNV) {
-        int nonempty = 0;
-        for (int c = 0; c < ncol; c++) nonempty += color_nonempty[c];
-        const i64 per_class = (nv + std::max(nonempty, 1) - 1) / std::max(nonempty, 1);
+    if (wblocks == 0 && nv <= kPersistMaxNV) {
         if (nv <= kDenseMaxNV || per_class <= kPersistMaxPerColor) {
             pblocks = persistent_blocks();
             // dense graphs: the grid's two halves take the color steps in turn
@@ -460,20 +475,6 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
                                               dense ? kPersistMaxBlocks : kPersistMaxBlocksHash});
                 if (dense) pblocks = std::max(2, pblocks & ~1);
             }
-        }
-    }
-    // large graphs: the whole-GPU persistent sweep (wide.hpp), plain form only
-    const bool las_mode = las && !(las->mode == 2 && nv <= kDenseMaxNV) && las->mode != 0;
-    int wblocks = 0;
-    {
-        int nonempty = 0;
-        for (int c = 0; c < ncol; c++) nonempty += color_nonempty[c];
-        // classes of more than kWideMaxPerColor vertices on average fill the GPU
-        // with per-color launches of the binned kernels
-        const bool small_classes = nonempty > 0 && nv / nonempty <= kWideMaxPerColor;
-        if (!las_mode && pblocks == 0 && nv > kPersistMaxNV && small_classes && wide_enabled()) {
-            wblocks = wide_blocks();
-            if (tune_.wide_blocks > 0) wblocks = std::min(wblocks, tune_.wide_blocks);
         }
     }
     bool use_wide = wblocks > 0;
@@ -673,9 +674,10 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         bool done_iter = false;
         if (use_wide) {
             launch_fill_i32((int32_t *)wbar.p, (i64)wbar.n, 0, s_);
-            Profiler::get().begin(K_WIDE, s_);
+            const int cls = nv > kPersistMaxNV ? K_WIDE : K_PERSIST;
+            Profiler::get().begin(cls, s_);
             use_wide = launch_wide_iteration(W, wblocks, s_);
-            Profiler::get().end(K_WIDE, 24.0 * g.nnz + 32.0 * nv, s_);
+            Profiler::get().end(cls, 24.0 * g.nnz + 32.0 * nv, s_);
             if (use_wide) {
                 launch_sum_partials(wpart.p, wblocks, res.p, s_);
                 launch_sum_partials(wpart.p + wblocks, wblocks, res.p + 1, s_);
@@ -800,7 +802,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         prevMod = currMod;
     }
     if (labels32) launch_widen_ids(wc0.p, nv, C, s_);
-    if (wmoves.n) moves_ += fetch(wmoves.p);
+    if (wmoves.n && nv > kPersistMaxNV) moves_ += fetch(wmoves.p);  // glv_stats::moves: large graphs only
     if (mode) sync();
     if (las_off) {
         las->swept_vertices += (i64)numItrs * nonisolated;

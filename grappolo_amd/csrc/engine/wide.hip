@@ -834,6 +834,13 @@ int wide_blocks() {
     return cached;
 }
 
+int wide_grid(i64 entries) {
+    const int most = wide_blocks();
+    int nb = kWMinGrid;
+    while (nb < most && (i64)nb * kWBlock < entries) nb *= 2;
+    return std::min(nb, most);
+}
+
 bool launch_wide_iteration(const WideArgs &W, int nblocks, hipStream_t s) {
     if (nblocks <= 0 || nblocks > wide_blocks()) return false;
     WideArgs w = W;

@@ -1,4 +1,5 @@
-// wide.hpp -- whole-GPU persistent colored iteration for large graphs.
+// wide.hpp -- whole-GPU persistent colored iteration for graphs above
+// kDenseMaxNV vertices.
 //
 // One launch per colored iteration (all color steps of the iteration, the
 // per-color loop of Coloring/parallelLouvainWithColoring.cpp:169-218 with the
@@ -142,6 +143,14 @@ bool build_wide_plan(const DevGraph &g, const PhaseSetup &P, int nb, WidePlan &L
 bool wide_enabled();
 // Resident workgroups of the wide sweep on the current device (0: unavailable).
 int wide_blocks();
+// The grid for color classes of `entries` adjacency entries on average: the
+// smallest power of two with a thread per entry, from kWMinGrid up to every
+// CU.  A larger grid lengthens each step's barrier, a smaller one its work;
+// measured (RMAT 100,001 vertices, 34k entries per class: first phase 25.9 ms
+// at 64 workgroups, 27.1 at 128, 28.5 at 32; RMAT 500,001, 103k: 112.6 ms at
+// 128, 118.8 at 256, 123.7 at 64; LFR 200,001, 290k: 6.5 ms at 256, 7.3 at 128).
+constexpr int kWMinGrid = 32;
+int wide_grid(i64 entries);
 // One colored iteration; false when the launch is not possible.
 bool launch_wide_iteration(const WideArgs &W, int nblocks, hipStream_t s);
 // (vertex, degree) of perm[lo .. hi) into vd[2 * (hi - lo)]

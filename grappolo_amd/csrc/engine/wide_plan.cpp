@@ -143,7 +143,9 @@ bool build_wide_plan(const DevGraph &g, const PhaseSetup &P, int nb, WidePlan &L
     }
     // the classes are planned independently, on host threads, then concatenated
     std::vector<ClassPlan> cp(ncol);
-    const int nthreads = (int)std::min<i64>(ncol, host_threads());
+    // (a thread per 16384 vertices: starting one costs about what planning
+    // that many does)
+    const int nthreads = (int)std::min<i64>({(i64)ncol, (i64)host_threads(), 1 + g.nv / 16384});
     std::atomic<int> next{0};
     std::atomic<bool> no_memory{false};
     auto worker = [&]() {

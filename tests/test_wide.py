@@ -90,3 +90,30 @@ def test_one_iteration_agrees_with_oracle(weighted):
         assert q == qo
     qg = oracle.modularity(g, got)
     assert abs(engine.modularity_dev(dg, C) - qg) <= 1e-12 * abs(qg)
+
+
+@pytest.mark.parametrize("valid", [True, False])
+@pytest.mark.parametrize("nv", [15360, 15361, 20000])
+def test_phase_on_both_sides_of_the_dense_limit(nv, valid):
+    """A whole colored phase at the vertex count where the whole-GPU sweep
+    takes over from the dense persistent one (15,360), with self-loops and
+    isolated vertices, a proper coloring and one whose classes hold edges:
+    labels, iterations and modularity equal the oracle's frozen color steps
+    (integer weights, so sums are exact in any order)."""
+    from grappolo_amd import engine
+    from grappolo_amd.graph import Graph, gen_planted
+    core = gen_planted(nv - 50, 20, 12, 0.25, seed=nv)
+    rows = np.repeat(np.arange(core.numVertices), core.degrees())
+    keep = rows < core.tails
+    loops = np.arange(0, core.numVertices, 11)
+    pairs = np.concatenate([np.stack([rows[keep], core.tails[keep]], 1), np.stack([loops, loops], 1)])
+    w = np.concatenate([np.ones(int(keep.sum())), np.full(len(loops), 2.0)])
+    g = Graph.from_pairs(nv, pairs, w)
+    colors, mc = oracle.color_greedy(g)
+    if not valid:
+        colors = (np.arange(nv) * 7 % 5).astype(np.int32)
+        mc = 4
+    q, C, it = engine.algoLouvainWithDistOneColoring(g, colors, mc + 1, -1.0, 1e-6)
+    qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+    assert it == ito and q == qo
+    np.testing.assert_array_equal(C, Co)
