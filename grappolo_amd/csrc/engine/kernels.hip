@@ -2753,7 +2753,8 @@ __device__ inline ChunkRows stage_rows(const i64 *off, const i64 *C, i64 nv, i64
     ChunkRows R{s_r[0], s_r[1], s_r[1] <= kCoarsenRows};
     if (R.staged) {
         for (i64 i = threadIdx.x; i <= R.nr; i += blockDim.x) s_off[i] = off[R.r0 + i];
-        for (i64 i = threadIdx.x; i < R.nr; i += blockDim.x) s_c[i] = C[R.r0 + i];
+        if (C)
+            for (i64 i = threadIdx.x; i < R.nr; i += blockDim.x) s_c[i] = C[R.r0 + i];
     }
     __syncthreads();
     return R;
@@ -2771,6 +2772,34 @@ __device__ inline i64 row_label(const ChunkRows &R, const i64 *s_off, const i64 
         return s_c[lo];
     }
     return C[row_of(off, R.r0, R.r0 + R.nr - 1, j)];
+}
+// The row of entry j (a chunk's rows staged, or searched in HBM).
+__device__ inline i64 row_index(const ChunkRows &R, const i64 *s_off, const i64 *off, i64 j) {
+    if (!R.staged) return row_of(off, R.r0, R.r0 + R.nr - 1, j);
+    int lo = 0, hi = (int)R.nr - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s_off[mid] <= j) lo = mid;
+        else hi = mid - 1;
+    }
+    return R.r0 + lo;
+}
+__global__ __launch_bounds__(kBlock) void k_entry_labels(const i64 *off, const i64 *tails, const double *w, i64 nv,
+                                                         i64 nnz, int32_t *lab, double *selfw) {
+    __shared__ i64 s_off[kCoarsenRows + 1], s_r[2];
+    const i64 nchunks = (nnz + kCoarsenChunk - 1) / kCoarsenChunk;
+    for (i64 ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
+        const i64 e0 = ch * kCoarsenChunk, e1 = e0 + kCoarsenChunk < nnz ? e0 + kCoarsenChunk : nnz;
+        const ChunkRows R = stage_rows(off, nullptr, nv, e0, e1, s_off, nullptr, s_r);
+        const i64 r1 = R.r0 + R.nr;
+        for (i64 j = e0 + threadIdx.x; j < e1; j += kBlock) {
+            const i64 t = tails[j];
+            lab[j] = (int32_t)t;
+            // only a neighbour among the chunk's own rows can be the row itself
+            if (t >= R.r0 && t < r1 && row_index(R, s_off, off, j) == t) atomicAdd(&selfw[t], w[j]);
+        }
+        __syncthreads();  // s_off is restaged
+    }
 }
 __global__ __launch_bounds__(kBlock) void k_coarsen_count(const i64 *off, const i64 *tails, const i64 *C, i64 nv,
                                                        i64 nnz, i64 *ccount) {
@@ -3428,6 +3457,42 @@ void sort_pairs_u32_i64(uint32_t *keys, i64 *vals, i64 n, int end_bit, hipStream
     GLV_HIP(rocprim::radix_sort_pairs(tmp.p, bytes, keys, k2.p, vals, v2.p, (size_t)n, 0, end_bit, s));
     GLV_HIP(hipMemcpyAsync(keys, k2.p, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     GLV_HIP(hipMemcpyAsync(vals, v2.p, n * sizeof(i64), hipMemcpyDeviceToDevice, s));
+}
+void launch_entry_labels(const DevGraph &g, int32_t *lab, double *selfw, hipStream_t s) {
+    launch_fill_f64(selfw, g.nv, 0.0, s);
+    const i64 nch = coarsen_chunks(g.nnz);
+    if (nch <= 0) return;
+    k_entry_labels<<<(unsigned)std::min<i64>(nch, 8192), kBlock, 0, s>>>(g.off, g.tails, g.w, g.nv, g.nnz, lab,
+                                                                         selfw);
+    GLV_LAUNCH_CHECK();
+}
+__global__ void k_positions(const int32_t *tails, i64 n, uint32_t *keys, uint32_t *pos) {
+    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
+        keys[i] = (uint32_t)tails[i];
+        pos[i] = (uint32_t)i;
+    }
+}
+void group_entries_by_tail(const DevGraph &g, const int32_t *tails32, DBuf<uint32_t> &pos, i64 *start,
+                           hipStream_t s) {
+    const i64 n = g.nnz;
+    pos.alloc(std::max<i64>(n, 1), s);
+    if (n <= 0) {
+        launch_fill_i64(start, g.nv + 1, 0, s);
+        return;
+    }
+    int bits = 1;
+    while (((i64)1 << bits) < g.nv) bits++;
+    DBuf<uint32_t> k0(n, s), k1(n, s), p1(n, s);
+    k_positions<<<grid_for(n, kBlock, 16384), kBlock, 0, s>>>(tails32, n, k0.p, pos.p);
+    GLV_LAUNCH_CHECK();
+    rocprim::double_buffer<uint32_t> kb(k0.p, k1.p), pb(pos.p, p1.p);
+    size_t bytes = 0;
+    GLV_HIP(rocprim::radix_sort_pairs(nullptr, bytes, kb, pb, (size_t)n, 0, bits, s));
+    DBuf<char> tmp(bytes, s);
+    GLV_HIP(rocprim::radix_sort_pairs(tmp.p, bytes, kb, pb, (size_t)n, 0, bits, s));
+    if (pb.current() != pos.p) std::swap(pos, p1);
+    k_slice_starts<<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(kb.current(), n, g.nv, start);
+    GLV_LAUNCH_CHECK();
 }
 void sort_pairs_u64_f64(u64 *keys, double *vals, i64 n, int end_bit, hipStream_t s) {
     if (n <= 1) return;

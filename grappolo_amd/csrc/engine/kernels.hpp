@@ -84,6 +84,15 @@ void launch_sum(const double *x, i64 n, double *part, double *out, hipStream_t s
 void launch_sumsq(const double *x, i64 n, double *part, double *out, hipStream_t s);
 void launch_sum_partials(const double *part, i64 np, double *out, hipStream_t s);
 
+// --- entry labels (whole-GPU sweep) ----------------------------------------
+// lab[j] = tails[j] as 32 bits; selfw[v] = the weight of v's self-loop entries
+void launch_entry_labels(const DevGraph &g, int32_t *lab, double *selfw, hipStream_t s);
+// the entries grouped by neighbour: pos[start[v] .. start[v + 1]) are the
+// positions j with tails[j] == v (g.nnz < 2^32); tails32: the neighbours as
+// launch_entry_labels wrote them
+void group_entries_by_tail(const DevGraph &g, const int32_t *tails32, DBuf<uint32_t> &pos, i64 *start,
+                           hipStream_t s);
+
 // --- sweeps --------------------------------------------------------------
 // number of block partials the sweep of `bin` writes for `count` vertices
 i64 sweep_blocks(int bin, i64 count, i64 nv);

@@ -510,7 +510,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     }
     DBuf<unsigned> bar(pblocks > 0 ? kBarrierWords : 0, s_);
     DBuf<double> ppart(pblocks > 0 ? 2 * pblocks : 0, s_);
-    if (use_wide && (nv >= (i64(1) << 31) || g.nnz >= (i64(1) << 40))) use_wide = false;  // 32-bit ids
+    if (use_wide && (nv >= (i64(1) << 31) || g.nnz >= (i64(1) << 32))) use_wide = false;  // 32-bit ids and positions
     const bool dbl = pblocks > 0 || use_wide;
     DBuf<i64> cperm(dbl ? nv : 0, s_), cstart(dbl ? ncol + 1 : 0, s_);
     // second state buffers of the persistent sweep (one grid barrier per color step)
@@ -525,32 +525,53 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     DBuf<double> wpart(use_wide ? 2 * (size_t)wblocks : 0, s_);
     DBuf<i64> wmoves(use_wide ? 1 : 0, s_);
     DBuf<CommInfo> wm0(use_wide ? nv : 0, s_), wm1(use_wide ? nv : 0, s_);
-    if (use_wide) use_wide = build_wide_plan(g, P, wblocks, WP, s_);
-    // the wide sweep's 32-bit labels (two buffers) and neighbour ids; while
-    // it runs, the phase's labels live in wc0 (copied back to C when a full
-    // modularity pass or the end of the phase needs them)
-    DBuf<int32_t> wc0(use_wide ? nv : 0, s_), wc1(use_wide ? nv : 0, s_), wtails(use_wide ? g.nnz : 0, s_);
+    // the wide sweep's 32-bit labels, the labels held per entry and the entry
+    // positions grouped by neighbour; while it runs, the phase's labels live in
+    // wc (copied back to C when a full modularity pass or the end of the phase
+    // needs them)
+    DBuf<int32_t> wlab(use_wide ? std::max<i64>(g.nnz, 1) : 0, s_);
+    DBuf<double> wself(use_wide ? nv : 0, s_);
+    if (use_wide) {
+        launch_entry_labels(g, wlab.p, wself.p, s_);
+        use_wide = build_wide_plan(g, P, wself.p, wblocks, WP, s_);
+    }
+    DBuf<int32_t> wc(use_wide ? nv : 0, s_), wtgt(use_wide ? nv : 0, s_);
+    DBuf<uint32_t> wtpos;
+    DBuf<i64> wtoff(use_wide ? nv + 1 : 0, s_);
     bool labels32 = false;
     if (use_wide) {
-        launch_narrow_ids(C, nv, wc0.p, s_);
-        launch_narrow_ids(g.tails, g.nnz, wtails.p, s_);
+        launch_narrow_ids(C, nv, wc.p, s_);
+        group_entries_by_tail(g, wlab.p, wtpos, wtoff.p, s_);
         labels32 = true;
         launch_fill_i64(wmoves.p, 1, 0, s_);
-        W.A = A;
-        W.C0 = wc0.p;
-        W.C1 = wc1.p;
-        W.tails = wtails.p;
+        W.w = g.w;
+        W.k = P.k.p;
+        W.constant = P.constant;
+        W.nv = nv;
+        W.C = wc.p;
+        W.tgt = wtgt.p;
+        W.lab = wlab.p;
+        W.tpos = wtpos.p;
+        W.toff = wtoff.p;
+        W.selfw = wself.p;
+        W.defer = !valid_colors;
         W.a = P.a.p;
         W.n = P.n.p;
         W.m0 = wm0.p;
         W.m1 = wm1.p;
-        W.perm = P.perm.p;
+        W.rows = WP.rows.p;
         W.cperm = cperm.p;
-        W.cstart = cstart.p;
+        W.classes = WP.classes.p;
+        W.ncls = WP.ncls;
+        W.over = WP.over.p;
+        W.rank = WP.rank.p;
         W.witems = WP.witems.p;
-        W.wstart = WP.wstart.p;
-        W.vitems = WP.vitems.p;
-        W.vstart = WP.vstart.p;
+        W.wbeg = WP.wbeg.p;
+        W.wend = WP.wend.p;
+        W.pitems = WP.pitems.p;
+        W.pbeg = WP.pbeg.p;
+        W.pend = WP.pend.p;
+        W.live = (int)nv;
         W.giants = WP.giants.p;
         W.ngiants = WP.ngiants;
         W.gpk = WP.gpk.p;
@@ -562,7 +583,6 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         W.gcid = WP.gcid.p;
         W.gparts = WP.gparts;
         W.gout = WP.gout.p;
-        W.ncol = ncol;
         W.bar = wbar.p;
         W.part = wpart.p;
         W.moves = wmoves.p;
@@ -682,17 +702,19 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
                 launch_sum_partials(wpart.p, wblocks, res.p, s_);
                 launch_sum_partials(wpart.p + wblocks, wblocks, res.p + 1, s_);
                 double h[2];
-                unsigned abort_flag = 0;
+                unsigned state[2] = {0, 0};  // abort flag, communities left
                 Readback rb(s_);
                 rb.add(h, res.p, sizeof(h));
-                rb.add(&abort_flag, wbar.p, sizeof(unsigned));
+                rb.add(state, wbar.p, sizeof(state));
                 rb.run();
+                const unsigned abort_flag = state[0];
+                W.live = (int)state[1];
                 if (abort_flag & 2)
                     fail(GLV_E_UNSUPPORTED, "a partition of a giant vertex's communities outgrew the LDS table");
                 if (abort_flag) fail(GLV_E_DEVICE, "grid barrier of the wide sweep timed out");
                 if (numItrs == 1 || !valid_colors) {
                     // a full pass: the first iteration, or classes that may hold an edge
-                    launch_widen_ids(wc0.p, nv, C, s_);
+                    launch_widen_ids(wc.p, nv, C, s_);
                     currMod = colored_modularity(g, P, C, part.p, res.p, &exx);
                 } else {
                     // moves of one color step are pairwise non-adjacent, so the
@@ -704,7 +726,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
                 done_iter = true;
             } else {
                 // launch refused: this phase continues with per-color launches
-                launch_widen_ids(wc0.p, nv, C, s_);
+                launch_widen_ids(wc.p, nv, C, s_);
                 labels32 = false;
             }
         }
@@ -801,7 +823,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         if (numItrs >= kMaxPhaseIters) break;
         prevMod = currMod;
     }
-    if (labels32) launch_widen_ids(wc0.p, nv, C, s_);
+    if (labels32) launch_widen_ids(wc.p, nv, C, s_);
     if (wmoves.n && nv > kPersistMaxNV) moves_ += fetch(wmoves.p);  // glv_stats::moves: large graphs only
     if (mode) sync();
     if (las_off) {

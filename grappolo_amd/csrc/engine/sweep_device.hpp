@@ -19,6 +19,23 @@ __device__ inline double ld_agent(const double *p) {
 __device__ inline i64 ld_agent(const i64 *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ inline int32_t ld_agent(const int32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline uint32_t ld_agent(const uint32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ inline void st_agent(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Waits for the calling wavefront's stores and atomics (s_waitcnt vmcnt(0));
+// the empty asm keeps the compiler from moving memory operations across.
+__device__ inline void stores_done() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    asm volatile("" ::: "memory");
+}
 
 // Gain of moving a vertex of degree kv from community s (internal weight
 // eix excluding its self-loop, degree ax excluding the vertex) to community y
@@ -139,12 +156,17 @@ constexpr unsigned kSpinLimit = 1u << 22;
 // 64 workgroups each lane polls every 64th slot.  bar holds 16 + 16 * nb words.
 // Bounded wait; a workgroup that gives up raises bar[0] (abort), which
 // releases every other wait.  Returns false when the barrier was abandoned.
-__device__ bool grid_barrier(unsigned *bar, unsigned nb, unsigned seq) {
-    __shared__ int s_ok;
-    unsigned *flags = bar + 16;  // flag of workgroup b at flags[16 * b]
+// The two halves of the barrier: between them a workgroup may do work that
+// neither reads what other workgroups write in this step nor writes memory.
+__device__ inline void grid_arrive(unsigned *bar, unsigned seq) {
+    stores_done();  // every wavefront's, before thread 0 releases them
     __syncthreads();
     if (threadIdx.x == 0)
-        __hip_atomic_store(&flags[16 * blockIdx.x], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&bar[16 + 16 * blockIdx.x], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline bool grid_wait(unsigned *bar, unsigned nb, unsigned seq) {
+    __shared__ int s_ok;
+    unsigned *flags = bar + 16;  // flag of workgroup b at flags[16 * b]
     if (threadIdx.x < kWave) {
         const int lane = threadIdx.x;
         unsigned spins = 0;
@@ -167,6 +189,10 @@ __device__ bool grid_barrier(unsigned *bar, unsigned nb, unsigned seq) {
     }
     __syncthreads();
     return s_ok != 0;
+}
+__device__ inline bool grid_barrier(unsigned *bar, unsigned nb, unsigned seq) {
+    grid_arrive(bar, seq);
+    return grid_wait(bar, nb, seq);
 }
 
 }  // namespace

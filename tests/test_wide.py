@@ -117,3 +117,41 @@ def test_phase_on_both_sides_of_the_dense_limit(nv, valid):
     qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
     assert it == ito and q == qo
     np.testing.assert_array_equal(C, Co)
+
+
+@pytest.mark.parametrize("stage", ["run", "phase"])
+def test_degrees_at_the_item_bounds(stage):
+    """Vertices whose entries sit at the bounds of the sweep's work items
+    (light / mid 64, mid / heavy 512 by way of bin 7's 256, heavy / giant
+    8192, one and several chunks of 4096, a table round past each) on a
+    planted background: the run's labels (labels pushed in the step; the
+    giants merged once few communities are left) and the stage entry point's
+    (pushed after the step, since it takes any colors) equal the oracle's."""
+    import torch
+    from grappolo_amd import engine
+    from grappolo_amd.graph import Graph, gen_planted
+    degrees = [64, 65, 255, 256, 257, 511, 512, 513, 1024, 1025, 4096, 4097, 8191, 8192, 8193, 12288, 12289, 20481]
+    nh, nv = len(degrees), 30000
+    core = gen_planted(nv - nh, 24, 8, 0.3, seed=4)
+    rows = np.repeat(np.arange(core.numVertices), core.degrees())
+    keep = rows < core.tails
+    pairs = [np.stack([rows[keep] + nh, core.tails[keep] + nh], 1)]
+    rng = np.random.default_rng(9)
+    for h, d in enumerate(degrees):
+        others = nh + rng.choice(nv - nh, size=d, replace=False)
+        pairs.append(np.stack([np.full(d, h), others], 1))
+    g = Graph.from_pairs(nv, np.concatenate(pairs))
+    assert g.degrees()[:nh].tolist() == degrees
+    if stage == "run":
+        dg = engine.DeviceGraph(g, "cuda")
+        C = torch.empty(nv, dtype=torch.int64, device="cuda")
+        st = engine.run_colored_dev(dg, C, minGraphSize=100, threshold=1e-9, C_threshold=1e-6)
+        Co, so = oracle.run_colored(g, coloring="jp", frozen=True, minGraphSize=100, threshold=1e-9, C_threshold=1e-6)
+        assert st["final_modularity"] == so["final_modularity"]
+        np.testing.assert_array_equal(C.cpu().numpy(), Co)
+    else:
+        colors, mc = oracle.color_greedy(g)
+        q, C, it = engine.algoLouvainWithDistOneColoring(g, colors, mc + 1, -1.0, 1e-6)
+        qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+        assert it == ito and q == qo
+        np.testing.assert_array_equal(C, Co)
