@@ -97,6 +97,47 @@ __global__ void k_sizes(const i64 *C, i64 n, i64 base, i64 nc, unsigned long lon
     }
 }
 
+// The same through counts in LDS, for at most kLdsSizes communities: device
+// atomics run at about 3.5e9/s whatever the address, so one per vertex took 605
+// us for 2,000,003 labels of 4000 communities; here a workgroup adds its
+// communities once (26 us).  The grid keeps those additions near 2^17.
+constexpr i64 kLdsSizes = 16384;
+constexpr int kSizesBlock = 1024;
+__global__ __launch_bounds__(kSizesBlock) void k_sizes_lds(const i64 *C, i64 n, i64 base, int nc,
+                                                           unsigned long long *sizes, int *err) {
+    extern __shared__ uint32_t cnt[];
+    for (int c = threadIdx.x; c < nc; c += kSizesBlock) cnt[c] = 0;
+    __syncthreads();
+    // (a workgroup counts fewer than 2^32 labels: see launch_sizes)
+    const i64 step = (i64)gridDim.x * kSizesBlock;
+    bool bad = false;
+    for (i64 i0 = blockIdx.x * (i64)kSizesBlock + threadIdx.x; i0 < n; i0 += 4 * step) {
+        i64 c[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) c[u] = i0 + u * step < n ? C[i0 + u * step] - base : -1;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (i0 + u * step >= n) continue;
+            if (c[u] < 0 || c[u] >= nc) bad = true;
+            else atomicAdd(&cnt[c[u]], 1u);
+        }
+    }
+    if (bad) atomicOr(err, 1);
+    __syncthreads();
+    for (int c = threadIdx.x; c < nc; c += kSizesBlock)
+        if (cnt[c]) atomicAdd(sizes + c, (unsigned long long)cnt[c]);
+}
+void launch_sizes(const i64 *C, i64 n, i64 base, i64 nc, i64 *sizes, int *err, hipStream_t s) {
+    unsigned long long *d = (unsigned long long *)sizes;
+    if (nc <= kLdsSizes && n < (i64(1) << 32)) {
+        const i64 blocks = std::min<i64>({std::max<i64>(16, 131072 / nc), 256, (n + kSizesBlock - 1) / kSizesBlock});
+        k_sizes_lds<<<(unsigned)blocks, kSizesBlock, nc * sizeof(uint32_t), s>>>(C, n, base, (int)nc, d, err);
+    } else {
+        k_sizes<<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(C, n, base, nc, d, err);
+    }
+    GLV_LAUNCH_CHECK();
+}
+
 __global__ void k_pair_keys(const i64 *C1, const i64 *C2, i64 n, i64 base1, i64 base2, i64 nc1, i64 nc2, u64 *keys,
                             int *err) {
     for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
@@ -147,20 +188,20 @@ struct LabelStats {
     int flags;
 };
 
-LabelStats label_stats(const i64 *C, i64 n, hipStream_t s) {
-    DBuf<unsigned long long> mx(1, s);
-    DBuf<int> fl(1, s);
-    GLV_HIP(hipMemsetAsync(mx.p, 0, sizeof(unsigned long long), s));
-    GLV_HIP(hipMemsetAsync(fl.p, 0, sizeof(int), s));
-    k_label_stats<<<grid_for(n, kCB, 2048), kCB, 0, s>>>(C, n, mx.p, fl.p);
+// of both labellings (one wait)
+void label_stats(const i64 *C1, const i64 *C2, i64 n, LabelStats r[2], hipStream_t s) {
+    DBuf<unsigned long long> d(4, s);  // maxima, then flags
+    launch_fill_i64((i64 *)d.p, 4, 0, s);
+    // (two same-address atomics a workgroup: a grid of 512)
+    k_label_stats<<<grid_for(n, kCB, 512), kCB, 0, s>>>(C1, n, d.p, (int *)(d.p + 2));
     GLV_LAUNCH_CHECK();
-    LabelStats r;
-    unsigned long long m = 0;
-    GLV_HIP(hipMemcpyAsync(&m, mx.p, sizeof(m), hipMemcpyDeviceToHost, s));
-    GLV_HIP(hipMemcpyAsync(&r.flags, fl.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    GLV_HIP(hipStreamSynchronize(s));
-    r.max = (i64)m - 1;
-    return r;
+    k_label_stats<<<grid_for(n, kCB, 512), kCB, 0, s>>>(C2, n, d.p + 1, (int *)(d.p + 3));
+    GLV_LAUNCH_CHECK();
+    unsigned long long h[4];
+    Readback rb(s);
+    rb.add(h, d.p, sizeof(h));
+    rb.run();
+    for (int q = 0; q < 2; q++) r[q] = LabelStats{(i64)h[q] - 1, (int)h[2 + q]};
 }
 
 void remap(i64 *C, i64 n, i64 from, i64 to, hipStream_t s) {
@@ -191,8 +232,8 @@ double gini_coefficient(i64 *d_sizes, i64 n, int numColors, hipStream_t s) {
             GLV_HIP(hipMemcpyAsync(d_sizes, tmp.p, n * sizeof(i64), hipMemcpyDeviceToDevice, s));
         }
         DBuf<unsigned long long> acc(2, s);
-        GLV_HIP(hipMemsetAsync(acc.p, 0, 2 * sizeof(unsigned long long), s));
-        k_gini_sums<<<grid_for(n, kCB, 2048), kCB, 0, s>>>(d_sizes, n, acc.p);
+        launch_fill_i64((i64 *)acc.p, 2, 0, s);
+        k_gini_sums<<<grid_for(n, kCB, 512), kCB, 0, s>>>(d_sizes, n, acc.p);
         GLV_LAUNCH_CHECK();
         unsigned long long h[2];
         GLV_HIP(hipMemcpyAsync(h, acc.p, sizeof(h), hipMemcpyDeviceToHost, s));
@@ -212,7 +253,9 @@ void compare_communities(i64 *C1, i64 *C2, i64 N, CompareResult &r, hipStream_t 
     if (!C1 || !C2) fail(GLV_E_INVALID_ARG, "null labels");
     r = CompareResult();
     // community counts and the -1 relabelling, :62-107
-    const LabelStats s1 = label_stats(C1, N, s), s2 = label_stats(C2, N, s);
+    LabelStats st[2];
+    label_stats(C1, C2, N, st, s);
+    const LabelStats s1 = st[0], s2 = st[1];
     if ((s1.flags | s2.flags) & 4) fail(GLV_E_INVALID_ARG, "label below -1");
     const bool zero1 = s1.flags & 1, zero2 = s2.flags & 1;
     i64 nC1 = s1.max + (zero1 ? 1 : 0);
@@ -234,21 +277,18 @@ void compare_communities(i64 *C1, i64 *C2, i64 N, CompareResult &r, hipStream_t 
     r.nC1 = nC1;
     r.nC2 = nC2;
 
-    DBuf<int> err(1, s);
-    GLV_HIP(hipMemsetAsync(err.p, 0, sizeof(int), s));
+    DBuf<unsigned long long> acc(4, s);  // pair sums, error flag
+    launch_fill_i64((i64 *)acc.p, 4, 0, s);
+    int *err = (int *)(acc.p + 3);
     // community sizes (the reference's clusterDist arrays) and sum C(size, 2)
     DBuf<i64> sz1(nC1, s), sz2(nC2, s);
     launch_fill_i64(sz1.p, nC1, 0, s);
     launch_fill_i64(sz2.p, nC2, 0, s);
-    k_sizes<<<grid_for(N, kBlock, 8192), kBlock, 0, s>>>(C1, N, base1, nC1, (unsigned long long *)sz1.p, err.p);
+    launch_sizes(C1, N, base1, nC1, sz1.p, err, s);
+    launch_sizes(C2, N, base2, nC2, sz2.p, err, s);
+    k_choose2<i64><<<grid_for(nC1, kCB, 512), kCB, 0, s>>>(sz1.p, nC1, acc.p + 0);
     GLV_LAUNCH_CHECK();
-    k_sizes<<<grid_for(N, kBlock, 8192), kBlock, 0, s>>>(C2, N, base2, nC2, (unsigned long long *)sz2.p, err.p);
-    GLV_LAUNCH_CHECK();
-    DBuf<unsigned long long> acc(3, s);
-    GLV_HIP(hipMemsetAsync(acc.p, 0, 3 * sizeof(unsigned long long), s));
-    k_choose2<i64><<<grid_for(nC1, kCB, 2048), kCB, 0, s>>>(sz1.p, nC1, acc.p + 0);
-    GLV_LAUNCH_CHECK();
-    k_choose2<i64><<<grid_for(nC2, kCB, 2048), kCB, 0, s>>>(sz2.p, nC2, acc.p + 1);
+    k_choose2<i64><<<grid_for(nC2, kCB, 512), kCB, 0, s>>>(sz2.p, nC2, acc.p + 1);
     GLV_LAUNCH_CHECK();
 
     // contingency cells: runs of the sorted pair keys
@@ -256,7 +296,7 @@ void compare_communities(i64 *C1, i64 *C2, i64 N, CompareResult &r, hipStream_t 
     if (kbits > 64) fail(GLV_E_UNSUPPORTED, "community counts too large for 64-bit pair keys");
     {
         DBuf<u64> keys(N, s), sorted(N, s);
-        k_pair_keys<<<grid_for(N, kBlock, 8192), kBlock, 0, s>>>(C1, C2, N, base1, base2, nC1, nC2, keys.p, err.p);
+        k_pair_keys<<<grid_for(N, kBlock, 8192), kBlock, 0, s>>>(C1, C2, N, base1, base2, nC1, nC2, keys.p, err);
         GLV_LAUNCH_CHECK();
         size_t bytes = 0;
         GLV_HIP(rocprim::radix_sort_keys(nullptr, bytes, keys.p, sorted.p, (size_t)N, 0, std::max(kbits, 1), s));
@@ -271,15 +311,14 @@ void compare_communities(i64 *C1, i64 *C2, i64 N, CompareResult &r, hipStream_t 
         DBuf<char> st(bytes, s);
         GLV_HIP(rocprim::run_length_encode(st.p, bytes, sorted.p, (size_t)N, uniq, counts.p, nruns.p, s));
         const i64 runs = fetch1(nruns.p, s);
-        k_choose2<i64><<<grid_for(runs, kCB, 2048), kCB, 0, s>>>(counts.p, runs, acc.p + 2);
+        k_choose2<i64><<<grid_for(runs, kCB, 512), kCB, 0, s>>>(counts.p, runs, acc.p + 2);
         GLV_LAUNCH_CHECK();
     }
-    unsigned long long h[3];
-    int e = 0;
-    GLV_HIP(hipMemcpyAsync(h, acc.p, sizeof(h), hipMemcpyDeviceToHost, s));
-    GLV_HIP(hipMemcpyAsync(&e, err.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    GLV_HIP(hipStreamSynchronize(s));
-    if (e) fail(GLV_E_INVALID_ARG, "label outside the community range");
+    unsigned long long h[4];
+    Readback rb(s);
+    rb.add(h, acc.p, sizeof(h));
+    rb.run();
+    if (h[3]) fail(GLV_E_INVALID_ARG, "label outside the community range");
     r.SameSame = (i64)h[2];
     r.Agree = r.SameSame;
     r.SameDiff = (i64)h[0] - r.SameSame;

@@ -96,3 +96,18 @@ def test_gini_equals_oracle(n):
     d = torch.from_numpy(sz).cuda()
     assert engine.gini_dev(d) == exp
     np.testing.assert_array_equal(d.cpu().numpy(), es)
+
+
+@pytest.mark.parametrize("nc", [1, 2, 1023, 16384, 16385, 40000])
+def test_sizes_on_both_sides_of_the_lds_limit(nc):
+    """Community sizes are counted in LDS up to 16,384 communities and with
+    device atomics above: counts and Gini coefficients equal the oracle's, and
+    a label past the last community is still refused."""
+    rng = np.random.default_rng(nc)
+    n = 50021
+    a, b = rng.integers(0, nc, n), rng.integers(0, max(nc // 2, 1), n)
+    a[0] = b[0] = 0
+    a[1] = nc - 1
+    exp, _, _ = oracle.compare(a, b)
+    got, _, _ = engine.computeCommunityComparisons(a, b)
+    _same(got, exp)
