@@ -264,13 +264,20 @@ void launch_coarsen_count(const DevGraph &g, const i64 *C, i64 *ccount, hipStrea
 // vf: no seeded self-loops and integer-truncated weights (buildNewGraphVF)
 void launch_coarsen_emit(const DevGraph &g, const i64 *C, const i64 *cbase, i64 k, int kb,
                          u64 *keys, double *vals, hipStream_t s, bool vf = false);
-// nself (nullable, zeroed): += number of self-loop keys
-void launch_coarsen_mirror(const u64 *ukeys, const double *uvals, i64 nu, int kb, u64 *keys,
-                           double *vals, hipStream_t s, i64 *nself = nullptr);
 // vertexFollowing: C[i] and *count (zeroed) += vertices to remove
 void launch_vertex_following(const DevGraph &g, i64 *C, i64 *count, hipStream_t s);
-void launch_coarsen_rows(const u64 *keys, const double *vals, i64 total, i64 k, int kb, i64 *off,
-                         i64 *tails, double *w, hipStream_t s);
+// The unique pairs (a, b), b <= a < k, of ukeys[0..nu) ((a << kb) | b, sorted;
+// nu < 2^32) in the orders the rows are built from: startl[r], startu[r] (k + 1
+// each) the pairs before row r's among the sorted pairs and among the pairs
+// a != b stably sorted by b (bkeys, idx); startu[k] of the latter in all.
+struct CoarsenOrders {
+    DBuf<i64> startl, startu;
+    DBuf<uint32_t> bkeys, idx;
+};
+void launch_coarsen_orders(const u64 *ukeys, i64 nu, i64 k, int kb, CoarsenOrders &O, hipStream_t s);
+// the symmetric graph of the pairs, rows sorted by tail: nu + startu[k] entries
+void launch_coarsen_rows(const u64 *ukeys, const double *usums, i64 nu, i64 k, int kb, const CoarsenOrders &O,
+                         i64 *off, i64 *tails, double *w, hipStream_t s);
 
 // --- AoS <-> SoA ---------------------------------------------------------
 void launch_split_edges(const void *aos, i64 nnz, i64 *tails, double *w, hipStream_t s);
@@ -283,7 +290,11 @@ void launch_check_graph(const i64 *off, const i64 *tails, i64 nv, i64 nnz, int32
 // exclusive prefix sum of in[0..n) into out[0..n); returns nothing, total = out[n-1]+in[n-1]
 void scan_exclusive_i64(const i64 *in, i64 *out, i64 n, hipStream_t s);
 void sort_pairs_u32_i64(uint32_t *keys, i64 *vals, i64 n, int end_bit, hipStream_t s);
-void sort_pairs_u64_f64(u64 *keys, double *vals, i64 n, int end_bit, hipStream_t s);
+// (stable; k0, v0 hold the sorted pairs on return, k1 and v1 are n scratch each)
+void sort_pairs_u64_f64(DBuf<u64> &k0, DBuf<u64> &k1, DBuf<double> &v0, DBuf<double> &v1, i64 n, int end_bit,
+                        hipStream_t s);
+void sort_pairs_u32_u32(DBuf<uint32_t> &k0, DBuf<uint32_t> &k1, DBuf<uint32_t> &v0, DBuf<uint32_t> &v1, i64 n,
+                        int end_bit, hipStream_t s);
 // returns number of unique keys (synchronises)
 i64 reduce_by_key_u64_f64(const u64 *keys, const double *vals, i64 n, u64 *ukeys, double *usums,
                           hipStream_t s);

@@ -1051,22 +1051,17 @@ void Engine::coarsen(const DevGraph &g, const i64 *C, i64 k, DevGraph &out, bool
     launch_coarsen_emit(g, C, pos.p, k, kb, keys.p, vals.p, s_, vf);
     cnt.release();
     pos.release();
-    sort_pairs_u64_f64(keys.p, vals.p, tot, 2 * kb, s_);
     DBuf<u64> ukeys(tot, s_);
     DBuf<double> usums(tot, s_);
+    sort_pairs_u64_f64(keys, ukeys, vals, usums, tot, 2 * kb, s_);
     const i64 nu = reduce_by_key_u64_f64(keys.p, vals.p, tot, ukeys.p, usums.p, s_);
     keys.release();
     vals.release();
-    DBuf<u64> k2(2 * nu, s_);
-    DBuf<double> v2(2 * nu, s_);
-    DBuf<i64> nself(1, s_);
-    launch_fill_i64(nself.p, 1, 0, s_);
-    launch_coarsen_mirror(ukeys.p, usums.p, nu, kb, k2.p, v2.p, s_, nself.p);
-    ukeys.release();
-    usums.release();
-    sort_pairs_u64_f64(k2.p, v2.p, 2 * nu, 2 * kb, s_);
+    if (nu >= (i64(1) << 32)) fail(GLV_E_UNSUPPORTED, "contracted graph of 2^32 pairs or more");
+    CoarsenOrders O;
+    launch_coarsen_orders(ukeys.p, nu, k, kb, O, s_);
     // self-loop entries appear once (k of them with the seeds)
-    const i64 total = 2 * nu - (vf ? fetch(nself.p) : k);
+    const i64 total = vf ? nu + fetch(O.startu.p + k) : 2 * nu - k;
     out.nv = k;
     out.nnz = total;
     out.num_edges = nu;  // NE_out + k (buildNextPhase.cpp:237)
@@ -1074,7 +1069,7 @@ void Engine::coarsen(const DevGraph &g, const i64 *C, i64 k, DevGraph &out, bool
     out.tails_buf.alloc(total, s_);
     out.w_buf.alloc(total, s_);
     out.adopt();
-    launch_coarsen_rows(k2.p, v2.p, total, k, kb, out.off_buf.p, out.tails_buf.p, out.w_buf.p, s_);
+    launch_coarsen_rows(ukeys.p, usums.p, nu, k, kb, O, out.off_buf.p, out.tails_buf.p, out.w_buf.p, s_);
     // B_coarsen = 24 nnz_in + 8 NV_in + 24 nnz_out + 8 (k+1)
     Profiler::get().end(K_COARSEN, 24.0 * g.nnz + 8.0 * nv + 24.0 * total + 8.0 * (k + 1), s_);
 }
