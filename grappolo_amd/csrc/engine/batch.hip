@@ -200,14 +200,20 @@ __global__ void k_mask_graphs(const i64 *vb, i64 ng, const uint8_t *keep, i64 *C
     }
 }
 
-// err |= 1 when an entry of graph g's rows points outside [vb[g], vb[g+1])
+// err |= 1 when an entry of graph g's rows points outside [vb[g], vb[g+1]); a
+// graph's entries are shared by gridDim.y workgroups (one each left the
+// largest of 128 graphs, 1.6M entries, 2.0 ms in a single workgroup)
+constexpr int kCheckSplit = 32;
 __global__ void k_check_blocks(const i64 *off, const i64 *tails, const i64 *vb, i64 ng, int32_t *err) {
+    const i64 step = (i64)gridDim.y * blockDim.x;
     for (i64 g = blockIdx.x; g < ng; g += gridDim.x) {
-        const i64 lo = vb[g], hi = vb[g + 1];
-        for (i64 j = off[lo] + threadIdx.x; j < off[hi]; j += blockDim.x) {
+        const i64 lo = vb[g], hi = vb[g + 1], end = off[hi];
+        bool bad = false;
+        for (i64 j = off[lo] + (i64)blockIdx.y * blockDim.x + threadIdx.x; j < end; j += step) {
             const i64 t = tails[j];
-            if (t < lo || t >= hi) atomicOr(err, 1);
+            bad = bad || t < lo || t >= hi;
         }
+        if (bad) atomicOr(err, 1);
     }
 }
 
@@ -217,7 +223,7 @@ __global__ void k_check_blocks(const i64 *off, const i64 *tails, const i64 *vb, 
 
 void launch_check_blocks(const i64 *off, const i64 *tails, const i64 *vb, i64 ng, int32_t *err, hipStream_t s) {
     if (ng <= 0) return;
-    k_check_blocks<<<(unsigned)std::max<i64>(1, std::min<i64>(ng, 65535)), kBB, 0, s>>>(off, tails, vb, ng, err);
+    k_check_blocks<<<dim3((unsigned)std::max<i64>(1, std::min<i64>(ng, 65535)), kCheckSplit), kBB, 0, s>>>(off, tails, vb, ng, err);
     GLV_LAUNCH_CHECK();
 }
 

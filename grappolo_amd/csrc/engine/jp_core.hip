@@ -408,7 +408,7 @@ void launch_jp_core(const i64 *hlist, i64 K, const i64 *loff, const int32_t *cor
 }
 void launch_jp_depth_max(const int32_t *dep, i64 nv, int32_t *maxd, hipStream_t s) {
     if (nv <= 0) return;
-    k_jp_depth_max<<<grid_for(nv, kBlock, 2048), kBlock, 0, s>>>(dep, nv, maxd);
+    k_jp_depth_max<<<grid_for(nv, kBlock, 256), kBlock, 0, s>>>(dep, nv, maxd);
     GLV_LAUNCH_CHECK();
 }
 void launch_jp_depth_hist(const int32_t *dep, i64 nv, int32_t top, unsigned *hist, hipStream_t s) {

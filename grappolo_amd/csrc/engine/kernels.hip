@@ -296,11 +296,26 @@ __global__ __launch_bounds__(kBlock) void k_red(const double *x, i64 n, double *
     s = block_sum(s);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
-__global__ __launch_bounds__(kBlock) void k_sum_partials(const double *part, i64 np, double *out) {
+// One workgroup, four loads in flight per thread: the partials' loads are its
+// whole time (18 us for 4096 partials one load at a time).
+constexpr int kSumBlock = 1024;
+__global__ __launch_bounds__(kSumBlock) void k_sum_partials(const double *part, i64 np, double *out) {
+    __shared__ double sh[kSumBlock / kWave];
     double s = 0;
-    for (i64 i = threadIdx.x; i < np; i += kBlock) s += part[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) out[0] = s;
+    for (i64 i0 = threadIdx.x; i0 < np; i0 += 4 * kSumBlock) {
+        double x[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) x[u] = i0 + u * kSumBlock < np ? part[i0 + u * kSumBlock] : 0.0;
+        s += (x[0] + x[1]) + (x[2] + x[3]);
+    }
+    s = wave_sum(s);
+    if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double r = 0;
+        for (int q = 0; q < kSumBlock / kWave; q++) r += sh[q];
+        out[0] = r;
+    }
 }
 
 // --------------------------------------------------------------------- sweeps
@@ -2663,11 +2678,16 @@ __global__ void k_jp_prio(const i64 *off, i64 nv, u64 *prio) {
     }
 }
 
-__global__ void k_jp_finish(const int32_t *colors, i64 nv, int32_t *maxc) {
+__global__ __launch_bounds__(kBlock) void k_jp_finish(const int32_t *colors, i64 nv, int32_t *maxc) {
+    __shared__ int s_m;
+    if (threadIdx.x == 0) s_m = -1;
+    __syncthreads();
     int m = -1;
     for (i64 v = blockIdx.x * (i64)blockDim.x + threadIdx.x; v < nv; v += (i64)gridDim.x * blockDim.x)
         m = colors[v] > m ? colors[v] : m;
-    atomicMax(maxc, m);
+    if (m >= 0) atomicMax(&s_m, m);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_m >= 0) atomicMax(maxc, s_m);
 }
 
 __global__ void k_color_conflicts(const i64 *off, const i64 *tails, i64 nv, const int32_t *colors,
@@ -2940,7 +2960,10 @@ __global__ __launch_bounds__(kBlock) void k_vertex_following(const i64 *off, con
         }
         C[i] = c;
     }
-    if (local) atomicAdd(count, local);
+    if (local) atomicAdd(&s_local, local);
+    __syncthreads();
+    // one device atomic per workgroup (one per thread serialised: 202 us at 1M vertices)
+    if (threadIdx.x == 0 && s_local) atomicAdd(count, (unsigned long long)s_local);
 }
 
 // ----------------------------------------------------------------- AoS/checks
@@ -3069,7 +3092,7 @@ void launch_sumsq(const double *x, i64 n, double *part, double *out, hipStream_t
     launch_sum_partials(part, kRedBlocks, out, s);
 }
 void launch_sum_partials(const double *part, i64 np, double *out, hipStream_t s) {
-    k_sum_partials<<<1, kBlock, 0, s>>>(part, np, out);
+    k_sum_partials<<<1, kSumBlock, 0, s>>>(part, np, out);
     GLV_LAUNCH_CHECK();
 }
 
@@ -3358,7 +3381,7 @@ void launch_jp_prio(const DevGraph &g, u64 *prio, hipStream_t s) {
 }
 void launch_jp_finish(int32_t *state, i64 nv, int32_t *maxc, hipStream_t s) {
     if (nv <= 0) return;
-    k_jp_finish<<<grid_for(nv, kBlock, 8192), kBlock, 0, s>>>(state, nv, maxc);
+    k_jp_finish<<<grid_for(nv, kBlock, 512), kBlock, 0, s>>>(state, nv, maxc);
     GLV_LAUNCH_CHECK();
 }
 void launch_color_conflicts(const DevGraph &g, const int32_t *colors, i64 *count, hipStream_t s) {
