@@ -13,6 +13,7 @@
 //   k_coarsen_*         buildNextLevelGraphOpt Utility/buildNextPhase.cpp:83-255
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include <rocprim/rocprim.hpp>
 
@@ -315,6 +316,142 @@ __global__ __launch_bounds__(kSumBlock) void k_sum_partials(const double *part, 
         double r = 0;
         for (int q = 0; q < kSumBlock / kWave; q++) r += sh[q];
         out[0] = r;
+    }
+}
+
+// ------------------------------------------------- modularity of a labelling
+// Per row, in vertex order, its weight (rk, nullable) and the weight of its
+// entries whose neighbour has the row's label (re): G lanes per row, so a
+// wavefront reads consecutive rows.  Neighbour labels are gathered from 32-bit
+// copies (LAB: read from the entry's label).  Rows of more than 64 G entries
+// are listed for k_row_sums_hub, a workgroup each.  The bound is the entry
+// stream (12 or 16 bytes each) and the gathers' L2 hits.
+template <int G, bool LAB>
+__global__ __launch_bounds__(kBlock) void k_row_sums(const i64 *off, const i64 *tails, const double *w,
+                                                     const int32_t *C, const int32_t *lab, i64 nv, double *rk,
+                                                     double *re, i64 *hubs, unsigned long long *nhubs) {
+    const int gl = threadIdx.x % G;
+    for (i64 v = (blockIdx.x * (i64)kBlock + threadIdx.x) / G; v < nv; v += (i64)gridDim.x * kBlock / G) {
+        const i64 beg = off[v], end = off[v + 1];
+        if (end - beg > 64 * G) {
+            if (gl == 0) hubs[atomicAdd(nhubs, 1ULL)] = v;
+            continue;
+        }
+        const int32_t s = C[v];
+        double k = 0, e = 0;
+        for (i64 j0 = beg + gl; j0 < end; j0 += 4 * G) {
+            double x[4];
+            int32_t c[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const i64 j = j0 + u * G;
+                x[u] = j < end ? w[j] : 0.0;
+                c[u] = j < end ? (LAB ? lab[j] : (int32_t)tails[j]) : -2;
+            }
+            if (!LAB) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) c[u] = c[u] >= 0 ? C[c[u]] : -2;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                k += x[u];
+                e += c[u] == s ? x[u] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) {
+            k += __shfl_xor(k, o, G);
+            e += __shfl_xor(e, o, G);
+        }
+        if (gl == 0) {
+            if (rk) rk[v] = k;
+            re[v] = e;
+        }
+    }
+}
+// sum over a workgroup of kSumBlock threads, in thread 0
+__device__ inline double sum_block(double s, double *sh) {
+    s = wave_sum(s);
+    __syncthreads();
+    if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = s;
+    __syncthreads();
+    double r = 0;
+    if (threadIdx.x == 0)
+        for (int q = 0; q < kSumBlock / kWave; q++) r += sh[q];
+    return r;
+}
+template <bool LAB>
+__global__ __launch_bounds__(kSumBlock) void k_row_sums_hub(const i64 *off, const i64 *tails, const double *w,
+                                                            const int32_t *C, const int32_t *lab, double *rk,
+                                                            double *re, const i64 *hubs,
+                                                            const unsigned long long *nhubs) {
+    __shared__ double sh[kSumBlock / kWave];
+    const i64 n = (i64)*nhubs;
+    for (i64 q = blockIdx.x; q < n; q += gridDim.x) {
+        const i64 v = hubs[q], end = off[v + 1];
+        const int32_t s = C[v];
+        double k = 0, e = 0;
+        for (i64 j = off[v] + threadIdx.x; j < end; j += kSumBlock) {
+            const double x = w[j];
+            k += x;
+            if ((LAB ? lab[j] : C[tails[j]]) == s) e += x;
+        }
+        k = sum_block(k, sh);
+        e = sum_block(e, sh);
+        if (threadIdx.x == 0) {
+            if (rk) rk[v] = k;
+            re[v] = e;
+        }
+    }
+}
+// a[C[v]] += x[v]: a wavefront adds up runs of equal labels first (vertices of
+// a community are often neighbours in the numbering, and same-address device
+// atomics serialise: 158 us for 1M vertices in runs of 64)
+__global__ __launch_bounds__(kBlock) void k_comm_degrees(const int32_t *C, const double *x, i64 nv, double *a) {
+    const int lane = threadIdx.x % kWave;
+    for (i64 i0 = blockIdx.x * (i64)kBlock + threadIdx.x - lane; i0 < nv; i0 += (i64)gridDim.x * kBlock) {
+        const i64 i = i0 + lane;
+        const int32_t c = i < nv ? C[i] : -1;
+        double t = i < nv ? x[i] : 0.0;
+        const int32_t cp = __shfl_up(c, 1), cn = __shfl_down(c, 1);
+        int head = lane == 0 || cp != c;
+        const bool last = lane == kWave - 1 || cn != c;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const double y = __shfl_up(t, o);
+            const int h = __shfl_up(head, o);
+            if (lane >= o && !head) {
+                t += y;
+                head = h;
+            }
+        }
+        if (last && c >= 0) atomicAdd(&a[c], t);
+    }
+}
+// block partials of sum rk, sum re and sum a^2 (kRedBlocks each), then k_mod_total
+__global__ __launch_bounds__(kSumBlock) void k_mod_partials(const double *rk, const double *re, const double *a,
+                                                            i64 nv, double *part) {
+    __shared__ double sh[kSumBlock / kWave];
+    double k = 0, e = 0, q = 0;
+    for (i64 i = blockIdx.x * (i64)kSumBlock + threadIdx.x; i < nv; i += (i64)gridDim.x * kSumBlock) {
+        if (rk) k += rk[i];
+        if (re) e += re[i];
+        if (a) q += a[i] * a[i];
+    }
+    k = sum_block(k, sh);
+    e = sum_block(e, sh);
+    q = sum_block(q, sh);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = k;
+        part[gridDim.x + blockIdx.x] = e;
+        part[2 * gridDim.x + blockIdx.x] = q;
+    }
+}
+__global__ __launch_bounds__(kSumBlock) void k_mod_total(const double *part, int np, double *out) {
+    __shared__ double sh[kSumBlock / kWave];
+    for (int f = 0; f < 3; f++) {
+        const double t = sum_block((int)threadIdx.x < np ? part[f * np + threadIdx.x] : 0.0, sh);
+        if (threadIdx.x == 0) out[f] = t;
     }
 }
 
@@ -3492,6 +3629,46 @@ void sort_pairs_u32_i64(uint32_t *keys, i64 *vals, i64 n, int end_bit, hipStream
     GLV_HIP(rocprim::radix_sort_pairs(tmp.p, bytes, keys, k2.p, vals, v2.p, (size_t)n, 0, end_bit, s));
     GLV_HIP(hipMemcpyAsync(keys, k2.p, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     GLV_HIP(hipMemcpyAsync(vals, v2.p, n * sizeof(i64), hipMemcpyDeviceToDevice, s));
+}
+template <bool LAB>
+static void row_sums(const DevGraph &g, const int32_t *C, const int32_t *lab, double *rk, double *re, hipStream_t s) {
+    DBuf<i64> hubs(g.nv, s);
+    DBuf<unsigned long long> nhubs(1, s);
+    launch_fill_i64((i64 *)nhubs.p, 1, 0, s);
+    // lanes per row: about half the mean degree
+    const i64 mean = g.nnz / g.nv;
+    auto go = [&](auto lanes) {
+        constexpr int G = decltype(lanes)::value;
+        k_row_sums<G, LAB><<<grid_for(g.nv * G, kBlock, 8192), kBlock, 0, s>>>(g.off, g.tails, g.w, C, lab, g.nv, rk,
+                                                                               re, hubs.p, nhubs.p);
+    };
+    if (mean <= 8) go(std::integral_constant<int, 4>());
+    else if (mean <= 16) go(std::integral_constant<int, 8>());
+    else if (mean <= 64) go(std::integral_constant<int, 16>());
+    else go(std::integral_constant<int, 64>());
+    GLV_LAUNCH_CHECK();
+    k_row_sums_hub<LAB><<<1024, kSumBlock, 0, s>>>(g.off, g.tails, g.w, C, lab, rk, re, hubs.p, nhubs.p);
+    GLV_LAUNCH_CHECK();
+}
+void launch_row_sums(const DevGraph &g, const int32_t *C, const int32_t *lab, double *rk, double *re,
+                     hipStream_t s) {
+    if (g.nv <= 0) return;
+    if (lab) row_sums<true>(g, C, lab, rk, re, s);
+    else row_sums<false>(g, C, lab, rk, re, s);
+}
+void launch_comm_degrees(const int32_t *C, const double *x, i64 nv, double *a, hipStream_t s) {
+    launch_fill_f64(a, nv, 0.0, s);
+    if (nv <= 0) return;
+    k_comm_degrees<<<grid_for(nv, kBlock, 4096), kBlock, 0, s>>>(C, x, nv, a);
+    GLV_LAUNCH_CHECK();
+}
+void launch_mod_sums(const double *rk, const double *re, const double *a, i64 nv, double *part, double *out,
+                     hipStream_t s) {
+    const int nb = (int)std::max<i64>(1, std::min<i64>(kModBlocks, (nv + kSumBlock - 1) / kSumBlock));
+    k_mod_partials<<<nb, kSumBlock, 0, s>>>(rk, re, a, nv, part);
+    GLV_LAUNCH_CHECK();
+    k_mod_total<<<1, kSumBlock, 0, s>>>(part, nb, out);
+    GLV_LAUNCH_CHECK();
 }
 void launch_entry_labels(const DevGraph &g, int32_t *lab, double *selfw, hipStream_t s) {
     launch_fill_f64(selfw, g.nv, 0.0, s);

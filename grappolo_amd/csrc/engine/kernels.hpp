@@ -84,6 +84,18 @@ void launch_sum(const double *x, i64 n, double *part, double *out, hipStream_t s
 void launch_sumsq(const double *x, i64 n, double *part, double *out, hipStream_t s);
 void launch_sum_partials(const double *part, i64 np, double *out, hipStream_t s);
 
+// --- modularity of a labelling --------------------------------------------
+// per row: its weight (rk, nullable) and its weight to its own community (re);
+// C: 32-bit labels; lab (nullable): the label of every entry's neighbour
+void launch_row_sums(const DevGraph &g, const int32_t *C, const int32_t *lab, double *rk, double *re,
+                     hipStream_t s);
+// a[c] = sum of x over the vertices labelled c (a: nv)
+void launch_comm_degrees(const int32_t *C, const double *x, i64 nv, double *a, hipStream_t s);
+// out[0..2] = sum rk, sum re, sum a^2 (each nullable); part: 3 * kModBlocks scratch
+constexpr int kModBlocks = 512;
+void launch_mod_sums(const double *rk, const double *re, const double *a, i64 nv, double *part, double *out,
+                     hipStream_t s);
+
 // --- entry labels (whole-GPU sweep) ----------------------------------------
 // lab[j] = tails[j] as 32 bits; selfw[v] = the weight of v's self-loop entries
 void launch_entry_labels(const DevGraph &g, int32_t *lab, double *selfw, hipStream_t s);

@@ -527,8 +527,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     DBuf<CommInfo> wm0(use_wide ? nv : 0, s_), wm1(use_wide ? nv : 0, s_);
     // the wide sweep's 32-bit labels, the labels held per entry and the entry
     // positions grouped by neighbour; while it runs, the phase's labels live in
-    // wc (copied back to C when a full modularity pass or the end of the phase
-    // needs them)
+    // wc (copied back to C at the end of the phase)
     DBuf<int32_t> wlab(use_wide ? std::max<i64>(g.nnz, 1) : 0, s_);
     DBuf<double> wself(use_wide ? nv : 0, s_);
     if (use_wide) {
@@ -536,6 +535,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         use_wide = build_wide_plan(g, P, wself.p, wblocks, WP, s_);
     }
     DBuf<int32_t> wc(use_wide ? nv : 0, s_), wtgt(use_wide ? nv : 0, s_);
+    DBuf<double> wre(use_wide ? nv : 0, s_), wmpart(use_wide ? 3 * kModBlocks : 0, s_), wmout(use_wide ? 3 : 0, s_);
     DBuf<uint32_t> wtpos;
     DBuf<i64> wtoff(use_wide ? nv + 1 : 0, s_);
     bool labels32 = false;
@@ -714,15 +714,18 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
                 if (abort_flag) fail(GLV_E_DEVICE, "grid barrier of the wide sweep timed out");
                 if (numItrs == 1 || !valid_colors) {
                     // a full pass: the first iteration, or classes that may hold an edge
-                    launch_widen_ids(wc.p, nv, C, s_);
-                    currMod = colored_modularity(g, P, C, part.p, res.p, &exx);
+                    Profiler::get().begin(K_MOD, s_);
+                    launch_row_sums(g, wc.p, wlab.p, nullptr, wre.p, s_);
+                    launch_mod_sums(nullptr, wre.p, nullptr, nv, wmpart.p, wmout.p, s_);
+                    Profiler::get().end(K_MOD, 24.0 * g.nnz + 16.0 * nv, s_);
+                    exx = fetch(wmout.p + 1);
                 } else {
                     // moves of one color step are pairwise non-adjacent, so the
                     // internal weight changes by the sum of the movers' 2(e_yt - e_ys)
                     exx += h[0];
-                    const double c = P.constant;
-                    currMod = exx * (double)c - h[1] * (double)c * (double)c;
                 }
+                const double c = P.constant;
+                currMod = exx * (double)c - h[1] * (double)c * (double)c;
                 done_iter = true;
             } else {
                 // launch refused: this phase continues with per-color launches
@@ -1075,6 +1078,22 @@ void Engine::coarsen(const DevGraph &g, const i64 *C, i64 k, DevGraph &out, bool
 }
 
 double Engine::modularity(const DevGraph &g, const i64 *C) {
+    if (g.nv < (i64(1) << 31)) {  // 32-bit labels: rows in vertex order, no grouping by degree
+        DBuf<int32_t> c32(g.nv, s_);
+        DBuf<double> rk(g.nv, s_), re(g.nv, s_), a(g.nv, s_), part(3 * kModBlocks, s_), out(3, s_);
+        Profiler::get().begin(K_MOD, s_);
+        launch_narrow_ids(C, g.nv, c32.p, s_);
+        launch_row_sums(g, c32.p, nullptr, rk.p, re.p, s_);
+        launch_comm_degrees(c32.p, rk.p, g.nv, a.p, s_);
+        launch_mod_sums(rk.p, re.p, a.p, g.nv, part.p, out.p, s_);
+        Profiler::get().end(K_MOD, 24.0 * g.nnz + 16.0 * g.nv, s_);
+        double h[3];
+        Readback rb(s_);
+        rb.add(h, out.p, sizeof(h));
+        rb.run();
+        const double c = (double)1 / h[0];
+        return h[1] * (double)c - h[2] * (double)c * (double)c;
+    }
     PhaseSetup P;
     setup(g, nullptr, 1, P);
     launch_comm_from_labels(C, P.k.p, g.nv, P.a.p, P.n.p, s_);

@@ -356,3 +356,27 @@ def test_colored_phase_set_aside_overflow(weighted):
         np.testing.assert_array_equal(C, Co)
     else:
         assert abs(q - qo) < 1e-3
+
+
+@pytest.mark.parametrize("mean", [2, 9, 20, 40, 120])
+def test_modularity_row_groups(mean):
+    """modularity_dev takes 4 to 64 lanes per row by mean degree and a workgroup
+    for rows beyond 64 entries a lane: labels in runs, scattered, -1 on
+    isolated vertices, with self-loops and rows at those bounds, against the
+    oracle (exact on integer weights)."""
+    import torch
+    nv = 4001
+    rng = np.random.default_rng(mean)
+    m = nv * mean // 2
+    pairs = [np.stack([rng.integers(20, nv - 30, m), rng.integers(20, nv - 30, m)], 1)]
+    for h, d in enumerate([255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 3900]):
+        pairs.append(np.stack([np.full(d, h), 20 + rng.choice(nv - 50, d, replace=False)], 1))
+    p = np.unique(np.sort(np.concatenate(pairs), 1), axis=0)
+    w = rng.integers(1, 9, len(p)).astype(np.float64)
+    from grappolo_amd.graph import Graph
+    g = Graph.from_pairs(nv, p, w)
+    dg = engine.DeviceGraph(g)
+    for C in (np.arange(nv) // 70, rng.integers(0, nv, nv), np.zeros(nv, np.int64)):
+        C = np.where(g.degrees() > 0, C, -1).astype(np.int64)
+        assert engine.modularity_dev(dg, torch.from_numpy(C).cuda()) == pytest.approx(oracle.modularity(g, C),
+                                                                                    rel=1e-14, abs=1e-15)
