@@ -442,18 +442,23 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     int nonempty = 0;
     for (int c = 0; c < ncol; c++) nonempty += color_nonempty[c];
     const i64 per_class = (nv + std::max(nonempty, 1) - 1) / std::max(nonempty, 1);
-    // graphs above the dense sweep's vertices: the whole-GPU persistent sweep
-    // (wide.hpp), plain form only.  Classes of more than kWideMaxPerColor
+    // graphs above the dense sweep's vertices, or whose classes are large: the
+    // whole-GPU persistent sweep (wide.hpp), plain form only.  Classes of more than kWideMaxPerColor
     // vertices on average fill the GPU with per-color launches of the binned
     // kernels.  Below 262,144 vertices it takes the place of those launches
     // and of the hash form of the persistent sweep: a 250,007-vertex RMAT run
     // went from 363 to 103 ms (its per-color launches took 13 ms per
     // iteration, most of it one HBM-table launch per class), a 62,103-vertex
-    // coarse phase of 69 colors from 45.2 to 14.9 ms; dense phases (<= 15,360
-    // vertices) are no faster here as long as their classes are small.
+    // coarse phase of 69 colors from 45.2 to 14.9 ms.  Dense phases (<= 15,360
+    // vertices) with classes of kWideDensePerColor vertices or more take it too
+    // (the dense sweep gives every vertex a workgroup of its own: a phase of
+    // 15,000 vertices and 9 colors 49.9 -> 8.0 ms, of 14,588 and 83 41.5 -> 23.2,
+    // of 1392 and 16 2.6 -> 2.4); with smaller classes the dense sweep's shorter
+    // steps win (1682 vertices, 50 colors: 5.9 ms against 7.1).
     const bool las_mode = las && !(las->mode == 2 && nv <= kDenseMaxNV) && las->mode != 0;
     int wblocks = 0;
-    if (!las_mode && nv > kDenseMaxNV && nonempty > 0 && nv / nonempty <= kWideMaxPerColor && wide_enabled()) {
+    if (!las_mode && (nv > kDenseMaxNV || per_class >= kWideDensePerColor) && nonempty > 0 &&
+        nv / nonempty <= kWideMaxPerColor && wide_enabled()) {
         wblocks = wide_grid(g.nnz / nonempty);
         if (tune_.wide_blocks > 0) wblocks = std::min(wblocks, tune_.wide_blocks);
     }

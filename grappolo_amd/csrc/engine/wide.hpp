@@ -1,5 +1,5 @@
 // wide.hpp -- whole-GPU persistent colored iteration for graphs above
-// kDenseMaxNV vertices.
+// kDenseMaxNV vertices and smaller ones with large color classes.
 //
 // One launch per colored iteration (all color steps of the iteration, the
 // per-color loop of Coloring/parallelLouvainWithColoring.cpp:169-218 with the
@@ -67,6 +67,9 @@ constexpr i64 kWMidMaxDeg = 512;         // largest vertex of a wavefront (load 
 // Phases whose color classes hold more vertices than this on average take the
 // per-color launches instead (a class that large fills the GPU by itself).
 constexpr i64 kWideMaxPerColor = 100000;
+// Phases of at most kDenseMaxNV vertices take the sweep from this many
+// vertices per color class on (the mean).
+constexpr i64 kWideDensePerColor = 64;
 
 // Relative costs of workgroup items (microseconds, measured order of
 // magnitude): a heavy vertex kWCostHeavy plus three per 1024 entries.

@@ -380,3 +380,28 @@ def test_modularity_row_groups(mean):
         C = np.where(g.degrees() > 0, C, -1).astype(np.int64)
         assert engine.modularity_dev(dg, torch.from_numpy(C).cuda()) == pytest.approx(oracle.modularity(g, C),
                                                                                     rel=1e-14, abs=1e-15)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_dense_sweep_sets_aside_with_small_classes(weighted):
+    """test_colored_phase_set_aside_overflow's blocks beside a clique, whose
+    colors bring the mean class below the size from which the whole-GPU sweep
+    takes a phase: the dense sweep gathers ahead, sets aside and overflows."""
+    from graphs import bipartite_blocks
+    from grappolo_amd.graph import Graph
+    b = bipartite_blocks(weighted=weighted)
+    rows = np.repeat(np.arange(b.numVertices), b.degrees())
+    keep = rows < b.tails
+    q = 60
+    iu = np.stack(np.triu_indices(q, 1), 1) + b.numVertices
+    g = Graph.from_pairs(b.numVertices + q, np.concatenate([np.stack([rows[keep], b.tails[keep]], 1), iu]),
+                         np.concatenate([b.weights[keep], np.ones(len(iu))]))
+    colors, mc, _ = oracle.color_jp(g)
+    assert g.numVertices / (mc + 1) < 64
+    q_, C, it = engine.algoLouvainWithDistOneColoring(g, colors.astype(np.int32), mc + 1, -1.0, 1e-6)
+    qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+    if not weighted:
+        assert it == ito and q_ == qo
+        np.testing.assert_array_equal(C, Co)
+    else:
+        assert abs(q_ - qo) < 1e-3
