@@ -2598,57 +2598,104 @@ __global__ __launch_bounds__(kBlock) void k_tail_prep(const i64 *off, const i64 
         }
     }
 }
-// Sequential first-fit over the n <= kJpTail tail vertices in list order, in
-// one workgroup with the bit rows in LDS: thread t holds the colour of tail
-// vertex t once it is chosen; vertex i's forbidden colours are base[i] plus
-// the colours of the set bits of row i.
-constexpr int kTailBatch = 8;  // base rows fetched together
-__global__ __launch_bounds__(kTailBlock) void k_tail_seq(const i64 *list, i64 n, i64 nv, const uint32_t *base,
-                                                         const u64 *adj, int32_t *colors, int32_t *err) {
-    constexpr int W = (int)(kJpTail / 64);
+// First-fit over the n <= kJpTail tail vertices in list order, in one
+// workgroup: thread t watches tail vertex t, which takes the first colour that
+// neither base[t] nor an earlier tail neighbour holds once all of those have
+// theirs -- the sequential result, in as many rounds as the longest chain of
+// earlier neighbours (a dozen in sparse tails, where one vertex after the
+// other took 0.55 us each).  A round: the ready vertices are listed, a
+// wavefront each gathers the neighbours' colours, two workgroup barriers.  In
+// LDS: the bit rows without the words no earlier vertex can be in, word-major
+// so that the threads' checks do not conflict, and the first kTailWords words
+// of the base rows (the rest is read from HBM when those are all taken).
+constexpr int kTailWords = 16;
+constexpr int kTailRows = (int)(kJpTail / 64);
+// word w of row t (t >= 64 w)
+__device__ inline int tail_word(int w, int t) { return w * (int)kJpTail - 32 * w * (w - 1) + t - 64 * w; }
+constexpr int kTailBits = kTailRows * (int)kJpTail - 32 * kTailRows * (kTailRows - 1);
+__global__ __launch_bounds__(kTailBlock) void k_tail_rounds(const i64 *list, int n, i64 nv, const uint32_t *base,
+                                                            const u64 *adj, int32_t *colors, int32_t *err) {
     constexpr int FW = kMaxColors / 32;
-    __shared__ u64 sadj[kJpTail * W];
-    __shared__ uint32_t forb[kTailBatch][FW];
-    __shared__ int s_cw[FW / kWave];
-    const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave;
-    for (i64 x = tid; x < n * W; x += kTailBlock) sadj[x] = adj[x];
-    int mine = 0;  // colour of tail vertex tid
-    for (int i0 = 0; i0 < n; i0 += kTailBatch) {
-        __syncthreads();  // the previous batch is done with forb
-        for (int x = tid; x < kTailBatch * FW; x += kTailBlock) {
-            const int r = i0 + x / FW;
-            forb[x / FW][x % FW] = r < n ? base[(i64)r * FW + x % FW] : 0u;
-        }
-        __syncthreads();
-        const int iend = (int)(i0 + kTailBatch < n ? i0 + kTailBatch : n);
-        for (int i = i0; i < iend; i++) {
-            const int r = i - i0;
-            if (tid < i && ((sadj[i * W + (tid >> 6)] >> (tid & 63)) & 1ull))
-                atomicOr(&forb[r][mine >> 5], 1u << (mine & 31));
-            __syncthreads();
-            int cw = kMaxColors;
-            if (tid < FW) {
-                const uint32_t m = forb[r][tid];
-                if (m != 0xFFFFFFFFu) cw = tid * 32 + __ffs((int)~m) - 1;
-            }
-#pragma unroll
-            for (int o = kWave / 2; o > 0; o >>= 1) {
-                const int x = __shfl_xor(cw, o);
-                cw = x < cw ? x : cw;
-            }
-            if (lane == 0 && w < FW / kWave) s_cw[w] = cw;
-            __syncthreads();
-            int c = kMaxColors;
-#pragma unroll
-            for (int q2 = 0; q2 < FW / kWave; q2++) c = s_cw[q2] < c ? s_cw[q2] : c;
-            if (c >= kMaxColors) {
-                if (tid == 0) atomicOr(err, 1);
-                c = 0;
-            }
-            if (tid == i) mine = c;
-        }
+    __shared__ u64 s_adj[kTailBits];
+    __shared__ uint32_t s_base[kJpTail * kTailWords];
+    __shared__ uint32_t s_forb[kTailBlock / kWave][FW];
+    __shared__ u64 s_done[kTailRows];
+    __shared__ uint16_t s_color[kJpTail], s_ready[kJpTail];
+    __shared__ int s_n[3];  // ready vertices, by round mod 3
+    const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
+    for (int x = t; x < n * kTailRows; x += kTailBlock) {
+        const int r = x / kTailRows, w = x % kTailRows;
+        if (64 * w <= r) s_adj[tail_word(w, r)] = adj[x];
     }
-    if (tid < n && list[tid] >= 0 && list[tid] < nv) colors[list[tid]] = mine;
+    for (int x = t; x < n * kTailWords; x += kTailBlock)
+        s_base[x] = base[(i64)(x / kTailWords) * FW + x % kTailWords];
+    if (t < kTailRows) s_done[t] = 0;
+    if (t < 3) s_n[t] = 0;
+    __syncthreads();
+    bool todo = t < n;
+    int at = 0;  // the first word of the row with a neighbour not yet coloured
+    for (int left = n, round = 0; left > 0; round = round == 2 ? 0 : round + 1) {
+        bool ready = todo;
+        if (todo)
+            for (; at <= t / 64; at++)
+                if (s_adj[tail_word(at, t)] & ~s_done[at]) {
+                    ready = false;
+                    break;
+                }
+        const u64 m = __ballot(ready);
+        int first = 0;
+        if (lane == 0 && m) first = atomicAdd(&s_n[round], __popcll(m));
+        first = __shfl(first, 0);
+        if (ready) s_ready[first + __popcll(m & ((1ULL << lane) - 1))] = (uint16_t)t;
+        todo = todo && !ready;
+        __syncthreads();
+        const int nr = s_n[round];  // at least one: the first uncoloured vertex is always ready
+        if (t == 0) s_n[round == 0 ? 2 : round - 1] = 0;  // (read before the last barrier)
+        for (int q = wv; q < nr; q += kTailBlock / kWave) {
+            const int v = s_ready[q];
+            uint32_t *forb = s_forb[wv];
+            int words = kTailWords, c = kMaxColors;
+            while (true) {
+                // the forbidden colours below 32 * words
+                for (int x = lane; x < words; x += kWave)
+                    forb[x] = x < kTailWords ? s_base[v * kTailWords + x] : base[(i64)v * FW + x];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                for (int w = 0; w <= v / 64; w++) {
+                    const u64 bits = s_adj[tail_word(w, v)];
+                    if ((bits >> lane) & 1) {
+                        const int cu = s_color[64 * w + lane];
+                        if (cu < 32 * words) atomicOr(&forb[cu >> 5], 1u << (cu & 31));
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                c = kMaxColors;
+                for (int x = lane; x < words; x += kWave) {
+                    const uint32_t f = forb[x];
+                    if (f != 0xFFFFFFFFu && c == kMaxColors) c = 32 * x + __ffs((int)~f) - 1;
+                }
+#pragma unroll
+                for (int o = kWave / 2; o > 0; o >>= 1) {
+                    const int x = __shfl_xor(c, o);
+                    c = x < c ? x : c;
+                }
+                if (c < kMaxColors || words == FW) break;
+                words = FW;
+            }
+            if (lane == 0) {
+                if (c >= kMaxColors) {
+                    atomicOr(err, 1);
+                    c = 0;
+                }
+                s_color[v] = (uint16_t)c;
+                atomicOr((unsigned long long *)&s_done[v >> 6], 1ULL << (v & 63));
+            }
+        }
+        left -= nr;
+        __syncthreads();
+    }
+    if (t < n && list[t] >= 0 && list[t] < nv) colors[list[t]] = s_color[t];
 }
 
 // Jones-Plassmann rounds in one persistent launch: the same topological
@@ -3484,7 +3531,7 @@ void launch_color_tail(const DevGraph &g, int32_t *state, i64 *flags, i64 *pos, 
     GLV_LAUNCH_CHECK();
     k_tail_prep<<<(unsigned)n, kBlock, 0, s>>>(g.off, g.tails, g.nv, state, list, tidx, base, adj);
     GLV_LAUNCH_CHECK();
-    k_tail_seq<<<1, kTailBlock, 0, s>>>(list, n, g.nv, base, adj, state, err);
+    k_tail_rounds<<<1, kTailBlock, 0, s>>>(list, (int)n, g.nv, base, adj, state, err);
     GLV_LAUNCH_CHECK();
 }
 int jp_persistent_blocks() {

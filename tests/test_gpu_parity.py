@@ -405,3 +405,27 @@ def test_dense_sweep_sets_aside_with_small_classes(weighted):
         np.testing.assert_array_equal(C, Co)
     else:
         assert abs(q_ - qo) < 1e-3
+
+
+@pytest.mark.parametrize("kind", ["clique", "path", "empty_rows", "dense"])
+def test_coloring_tail_rounds(kind):
+    """The tail's first-fit in rounds equals the sequential one: a clique of
+    1100 (every round one vertex, colors beyond the 512 held in LDS), a path
+    (chains in id order), tails of 1 to 1024 vertices, a dense random graph."""
+    from grappolo_amd.graph import Graph
+    rng = np.random.default_rng(3)
+    if kind == "clique":
+        graphs = [Graph.from_pairs(1100, np.stack(np.triu_indices(1100, 1), 1))]
+    elif kind == "path":
+        graphs = [Graph.from_pairs(n, np.stack([np.arange(n - 1), np.arange(1, n)], 1)) for n in (2, 64, 65, 1025)]
+    elif kind == "empty_rows":
+        graphs = [Graph.from_pairs(2000, np.array([[5, 1999]])),
+                  Graph.from_pairs(1300, np.stack([np.full(1299, 1299), np.arange(1299)], 1))]
+    else:
+        iu = np.stack(np.triu_indices(1500, 1), 1)
+        graphs = [Graph.from_pairs(1500, iu[rng.random(len(iu)) < p]) for p in (0.02, 0.3)]
+    for g in graphs:
+        c, mc = engine.algoDistanceOneVertexColoringOpt(g)
+        ref, rmc, _ = oracle.color_jp(g)
+        assert mc == rmc
+        np.testing.assert_array_equal(c, ref)
