@@ -39,10 +39,9 @@ void launch_graph_const(const i64 *vb, i64 ng, const double *k, double *gconst, 
 // skip: nothing to do when *skip is set (after every graph's phase has ended)
 void launch_graph_mod(const i64 *vb, i64 ng, const uint8_t *active, const double *eii, const double *a,
                       double *exx, double *a2, hipStream_t s, const int32_t *skip = nullptr);
-void launch_batch_decide(i64 ng, const double *exx, const double *a2, const double *gconst, const double *lower,
-                         double thresh, int maxitr, double *prev, double *curr, int32_t *itrs, uint8_t *active,
-                         uint8_t *apply, hipStream_t s);
-void launch_level_status(const i64 *vb, i64 ng, const uint8_t *active, int32_t *done, i64 *live, hipStream_t s);
+void launch_batch_decide(const i64 *vb, i64 ng, const double *exx, const double *a2, const double *gconst,
+                         const double *lower, double thresh, int maxitr, double *prev, double *curr, int32_t *itrs,
+                         uint8_t *active, uint8_t *apply, int32_t *done, i64 *live, hipStream_t s);
 void launch_batch_apply(i64 nv, const int32_t *gid, const uint8_t *apply, const i64 *tgt, i64 *curr, i64 *past,
                         const double *k, double *a, i64 *n, hipStream_t s, const int32_t *skip = nullptr);
 void launch_compact_graphs(const i64 *list, i64 n, const int32_t *gid, const uint8_t *active, const i64 *start,

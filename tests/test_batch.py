@@ -59,6 +59,26 @@ def test_batch_equals_separate_runs(basic_opt):
         assert res["final_clusters"][i] == st["final_clusters"], i
 
 
+@pytest.mark.parametrize("ng", [2048, 2049])
+def test_batch_of_many_graphs(ng):
+    """The largest batch whose graphs are decided in one launch with the
+    level's status, and the smallest decided by a grid of its own."""
+    import torch
+    from grappolo_amd import engine
+    kinds = [gen_planted(n, 2, 5.0, 0.2, seed=n) for n in (12, 20, 33)]
+    U, vb = union([kinds[i % 3] for i in range(ng)])
+    dg = engine.DeviceGraph(U, "cuda")
+    C = torch.empty(U.numVertices, dtype=torch.int64, device="cuda")
+    res = engine.run_basic_batch_dev(dg, vb, C)
+    Cb = C.cpu().numpy()
+    alone = [_standalone(g, 0) for g in kinds]
+    for i in range(ng):
+        Ci, st = alone[i % 3]
+        np.testing.assert_array_equal(Cb[vb[i]:vb[i + 1]], Ci, err_msg=f"graph {i}")
+        assert res["total_iterations"][i] == st["total_iterations"], i
+        assert res["final_modularity"][i] == st["final_modularity"], i
+
+
 def test_batch_weighted_within_tolerance():
     import torch
     from grappolo_amd import engine
