@@ -221,35 +221,39 @@ __global__ void k_slice_nnz(const i64 *start, const i64 *dscan, const i64 *degp,
     }
 }
 
-// sumVertexDegree: one thread per row sums in row order (the reference's
-// order) for rows up to 2048 entries; longer rows use a workgroup each.
-// k[v] = its weights summed in adjacency order (vertices of at most 2048
-// entries; the rest go to k_degree_big), one thread per row: for graphs of
-// high mean degree.
-__global__ void k_degree_rows_seq(const i64 *off, const double *w, i64 nv, double *k) {
-    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < nv; i += (i64)gridDim.x * blockDim.x) {
-        const i64 b = off[i], e = off[i + 1];
-        if (e - b > kBinMaxDeg[7]) continue;
-        double s = 0;
-        for (i64 j = b; j < e; j++) s += w[j];
-        k[i] = s;
-    }
-}
-// The same for graphs of low mean degree: a workgroup takes kBlock
+// sumVertexDegree: rows of up to 2048 entries are summed in row order (the
+// reference's order), longer rows use a workgroup each (k_degree_big).
+// k[v] of the short rows (at most `cut` entries): a workgroup takes kBlock
 // consecutive rows, streams their entries through LDS in coalesced tiles and
-// each thread adds its row's part of every tile in order.
+// each thread adds its row's part of every tile in order.  A tile takes the
+// time of the longest row in it, added up by one thread, and an RMAT graph has
+// its hubs side by side: with rows of up to 2048 entries here and the longer
+// ones streamed past, the phases of a 250,000-vertex graph took 4.0 ms, 0.36 ms
+// with k_degree_wave now.
 constexpr int kDegTile = 2048;
-constexpr i64 kDegTiledMean = 64;  // mean degree up to which the tiled form is used
-__global__ __launch_bounds__(kBlock) void k_degree_rows(const i64 *off, const double *w, i64 nv, double *k) {
+__global__ __launch_bounds__(kBlock) void k_degree_short(const i64 *off, const double *w, i64 nv, i64 cut, double *k) {
     __shared__ double tile[kDegTile];
+    __shared__ i64 s_off[kBlock + 1];
     for (i64 r0 = (i64)blockIdx.x * kBlock; r0 < nv; r0 += (i64)gridDim.x * kBlock) {
         const i64 r = r0 + threadIdx.x;
         const i64 rb = r < nv ? off[r] : 0, re = r < nv ? off[r + 1] : 0;
-        const bool mine = r < nv && re - rb <= kBinMaxDeg[7];
-        const i64 e0 = off[r0], e1 = off[r0 + kBlock < nv ? r0 + kBlock : nv];
+        const bool mine = r < nv && re - rb <= cut;
+        const int rows = (int)(nv - r0 < kBlock ? nv - r0 : kBlock);
+        __syncthreads();  // s_off and the last tile are read
+        if (r < nv) s_off[threadIdx.x] = rb;
+        if ((int)threadIdx.x == rows - 1) s_off[rows] = re;
+        __syncthreads();
+        const i64 e1 = s_off[rows];
         double acc = 0;
-        for (i64 t0 = e0; t0 < e1; t0 += kDegTile) {
-            const i64 t1 = t0 + kDegTile < e1 ? t0 + kDegTile : e1;
+        int cr = 0;  // the row of entry t0
+        i64 t1 = 0;
+        for (i64 t0 = s_off[0]; t0 < e1; t0 = t1) {
+            while (s_off[cr + 1] <= t0) cr++;
+            if (s_off[cr + 1] - s_off[cr] > cut) {  // not this kernel's: skipped
+                t1 = s_off[cr + 1];
+                continue;
+            }
+            t1 = t0 + kDegTile < e1 ? t0 + kDegTile : e1;
             __syncthreads();  // the previous tile is read
             for (i64 j = t0 + threadIdx.x; j < t1; j += kBlock) tile[j - t0] = w[j];
             __syncthreads();
@@ -259,6 +263,29 @@ __global__ __launch_bounds__(kBlock) void k_degree_rows(const i64 *off, const do
             }
         }
         if (mine) k[r] = acc;
+    }
+}
+// The same for the listed rows of up to 2048 entries, a wavefront per row: 64
+// entries are loaded together and added one lane after the other (the coarse
+// phases of a 1M-vertex LFR graph, mean degrees above 64: 1.1 ms with a thread
+// per row, whose loads are not coalesced, 0.23 ms so).
+__global__ __launch_bounds__(kBlock) void k_degree_wave(const i64 *off, const double *w, const i64 *verts, i64 count,
+                                                        double *k) {
+    const int lane = threadIdx.x % kWave;
+    const i64 nw = (i64)gridDim.x * (kBlock / kWave);
+    for (i64 q = blockIdx.x * (i64)(kBlock / kWave) + threadIdx.x / kWave; q < count; q += nw) {
+        const i64 v = verts[q], b = off[v], e = off[v + 1];
+        double s = 0;
+        double x = b + lane < e ? w[b + lane] : 0.0;
+        for (i64 j = b; j < e; j += kWave) {
+            const double nx = j + kWave + lane < e ? w[j + kWave + lane] : 0.0;  // the next 64 in flight
+            const int lo = __double2loint(x), hi = __double2hiint(x);
+#pragma unroll 16
+            for (int l = 0; l < kWave; l++)  // lanes past the end hold 0
+                s += __hiloint2double(__builtin_amdgcn_readlane(hi, l), __builtin_amdgcn_readlane(lo, l));
+            x = nx;
+        }
+        if (lane == 0) k[v] = s;
     }
 }
 __global__ void k_degree_big(const i64 *off, const double *w, const i64 *verts, i64 count, double *k) {
@@ -3260,13 +3287,17 @@ void launch_slices(const uint32_t *sorted_keys, const i64 *perm, const i64 *off,
     k_slice_nnz<<<grid_for(nkeys, kBlock, 8192), kBlock, 0, s>>>(start, dscan.p, degp.p, n, nkeys, pnnz);
     GLV_LAUNCH_CHECK();
 }
-void launch_degree(const DevGraph &g, const i64 *big, i64 nbig, double *k, hipStream_t s) {
+void launch_degree(const DevGraph &g, i64 cut, const i64 *mid, i64 nmid, const i64 *big, i64 nbig, double *k,
+                   hipStream_t s) {
     if (g.nv <= 0) return;
-    if (g.nnz <= kDegTiledMean * g.nv)
-        k_degree_rows<<<grid_for(g.nv, kBlock, 8192), kBlock, 0, s>>>(g.off, g.w, g.nv, k);
-    else
-        k_degree_rows_seq<<<grid_for(g.nv, kBlock, 8192), kBlock, 0, s>>>(g.off, g.w, g.nv, k);
-    GLV_LAUNCH_CHECK();
+    if (nmid + nbig < g.nv) {
+        k_degree_short<<<grid_for(g.nv, kBlock, 8192), kBlock, 0, s>>>(g.off, g.w, g.nv, cut, k);
+        GLV_LAUNCH_CHECK();
+    }
+    if (nmid > 0) {
+        k_degree_wave<<<grid_for(nmid, kBlock / kWave, 8192), kBlock, 0, s>>>(g.off, g.w, mid, nmid, k);
+        GLV_LAUNCH_CHECK();
+    }
     if (nbig > 0) {
         k_degree_big<<<(unsigned)std::min<i64>(nbig, 4096), kBlock, 0, s>>>(g.off, g.w, big, nbig, k);
         GLV_LAUNCH_CHECK();

@@ -96,7 +96,9 @@ void Engine::setup(const DevGraph &g, const int32_t *colors, int ncol, PhaseSetu
     }
     // degrees and 1/(2m)
     const i64 big_lo = P.bin_lo(8), big_hi = P.bin_hi(9);
-    launch_degree(g, P.perm.p + big_lo, big_hi - big_lo, P.k.p, s_);
+    const i64 mid_lo = P.bin_lo(6);
+    launch_degree(g, bins_.max_deg[5], P.perm.p + mid_lo, big_lo - mid_lo, P.perm.p + big_lo, big_hi - big_lo, P.k.p,
+                  s_);
     DBuf<double> part(kRedBlocks, s_), res(1, s_);
     launch_sum(P.k.p, nv, part.p, res.p, s_);
     P.total_weight = fetch(res.p);

@@ -429,3 +429,32 @@ def test_coloring_tail_rounds(kind):
         ref, rmc, _ = oracle.color_jp(g)
         assert mc == rmc
         np.testing.assert_array_equal(c, ref)
+
+
+@pytest.mark.parametrize("low", [False, True])
+def test_degree_sums_across_row_lengths(low):
+    """Weighted degrees of short rows (summed in tiles), rows of 65 to 2048
+    entries (a wavefront each) and longer ones (a workgroup each), side by side
+    and at the limits, with and without runs of short rows between them; with
+    the short bins lowered the limit moves with them.  Integer weights: the
+    sums are exact and the labels equal the oracle's."""
+    nv, rng = 6000, np.random.default_rng(2)
+    hubs = [1, 63, 64, 65, 2047, 2048, 2049, 64, 4200, 65, 1, 2048, 300]
+    first = np.concatenate([np.arange(len(hubs)), 256 + 3 * np.arange(len(hubs))])
+    rest = np.setdiff1d(np.arange(nv), first)
+    pairs = [np.stack([np.full(d, h), rng.choice(rest, d, replace=False)], 1) for h, d in zip(first, hubs + hubs)]
+    pairs = np.concatenate(pairs + [np.stack([rest[:-1], rest[1:]], 1)])
+    g = Graph.from_pairs(nv, pairs, rng.integers(1, 8, len(pairs)).astype(np.float64))
+    np.testing.assert_array_equal(g.degrees()[first], hubs + hubs)
+    bins = engine.get_bins()
+    try:
+        if low:
+            b = bins.copy()
+            b[3:6] = 8  # rows of more than 8 entries leave the tiles
+            engine.set_bins(b)
+        C, st = engine.runMultiPhaseBasic(g)
+    finally:
+        engine.set_bins(bins)
+    Co, so = oracle.run_basic(g)
+    np.testing.assert_array_equal(C, Co)
+    assert st["final_modularity"] == so["final_modularity"]
