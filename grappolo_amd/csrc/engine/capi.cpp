@@ -850,10 +850,10 @@ int glv_mlp_grad_dev(const float *d_params, const uint16_t *d_feats, const uint8
         B.n = n;
         B.batch = n;
         B.pos_weight = pos_weight;
-        const i64 nw = glv::mlp_grad_waves(n);
-        glv::DBuf<float> gpart(nw * glv::kMlpStride, s);
+        const i64 rows = glv::mlp_grad_rows(n);
+        glv::DBuf<float> gpart(rows * glv::kMlpStride, s);
         glv::launch_mlp_grad_partials(d_params, B, gpart.p, s);
-        glv::launch_mlp_reduce(gpart.p, nw, d_grad, s);
+        glv::launch_mlp_reduce(gpart.p, rows, d_grad, s);
         GLV_HIP(hipStreamSynchronize(s));
     });
 }
@@ -874,8 +874,8 @@ int glv_mlp_train_dev(float *d_params, float *d_m, float *d_v, const uint16_t *d
         B.random = 1;
         B.seed = seed;
         B.pos_weight = pos_weight;
-        const i64 nw = glv::mlp_grad_waves(batch);
-        glv::DBuf<float> gpart(nw * glv::kMlpStride, s);
+        const i64 rows = glv::mlp_grad_rows(batch);
+        glv::DBuf<float> gpart(rows * glv::kMlpStride, s);
         const double b1 = 0.9, b2 = 0.999;
         for (int64_t t = 0; t < steps; t++) {
             B.step = step0 + t;
@@ -883,7 +883,7 @@ int glv_mlp_train_dev(float *d_params, float *d_m, float *d_v, const uint16_t *d
             const float c1 = (float)(1.0 / (1.0 - std::pow(b1, k)));
             const float c2 = (float)(1.0 / (1.0 - std::pow(b2, k)));
             glv::launch_mlp_grad_partials(d_params, B, gpart.p, s);
-            glv::launch_mlp_adam(d_params, d_m, d_v, gpart.p, nw, lr, (float)b1, (float)b2, 1e-8f, c1, c2,
+            glv::launch_mlp_adam(d_params, d_m, d_v, gpart.p, rows, lr, (float)b1, (float)b2, 1e-8f, c1, c2,
                                  d_losses ? d_losses + t : nullptr, s);
         }
         GLV_HIP(hipStreamSynchronize(s));

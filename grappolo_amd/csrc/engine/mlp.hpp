@@ -29,9 +29,9 @@ constexpr int kMlpB2 = kMlpW2 + kMlpHidden * kMlpHidden;  // 4672
 constexpr int kMlpW3 = kMlpB2 + kMlpHidden;               // 4736
 constexpr int kMlpB3 = kMlpW3 + kMlpHidden;               // 4800
 constexpr int kMlpParams = kMlpB3 + 1;                    // 4801
-// per-wavefront gradient partial rows: params, then the loss
+// per-workgroup gradient partial rows: params, then the loss
 constexpr int kMlpStride = 4864;
-constexpr int kMlpMaxWaves = 512;
+constexpr int kMlpMaxRows = 512;  // two workgroups per CU
 
 // A batch of training samples.  random=0: sample j of the batch is j (the
 // batch is the first `batch` samples); random=1: it is
@@ -49,15 +49,15 @@ struct MlpBatch {
 
 // logits[i] of feats[i], i < n
 void launch_mlp_forward(const float *P, const uint16_t *feats, i64 n, float *logits, hipStream_t s);
-// number of wavefronts (partial rows) a gradient of `batch` samples uses
-i64 mlp_grad_waves(i64 batch);
-// per-wavefront partial gradients of the batch into gpart[w][kMlpStride]
+// number of workgroups (partial rows) a gradient of `batch` samples uses
+i64 mlp_grad_rows(i64 batch);
+// per-workgroup partial gradients of the batch into gpart[w][kMlpStride]
 void launch_mlp_grad_partials(const float *P, const MlpBatch &B, float *gpart, hipStream_t s);
-// grad[0..kMlpParams) and grad[kMlpParams] = loss, summed over nw partial rows in order
-void launch_mlp_reduce(const float *gpart, i64 nw, float *grad, hipStream_t s);
+// grad[0..kMlpParams) and grad[kMlpParams] = loss, summed over the partial rows in a fixed order
+void launch_mlp_reduce(const float *gpart, i64 nrows, float *grad, hipStream_t s);
 // reduce the partials, then one Adam step on P with moments m, v; loss of the
 // step into *loss when non-null.  c1, c2: bias corrections 1/(1-beta^t).
-void launch_mlp_adam(float *P, float *m, float *v, const float *gpart, i64 nw, float lr, float beta1,
+void launch_mlp_adam(float *P, float *m, float *v, const float *gpart, i64 nrows, float lr, float beta1,
                      float beta2, float eps, float c1, float c2, float *loss, hipStream_t s);
 
 }  // namespace glv

@@ -28,6 +28,15 @@ __device__ inline uint16_t bf16_bits(float f) {
     u += 0x7fffu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
 }
+// The same by the conversion instruction (one for two values; the integer form
+// takes eight operations each).  Of the 2^32 inputs only the 126 signalling NaNs
+// that BF16 can hold differ, which come out quiet; no arithmetic produces one.
+__device__ inline uint16_t bf16_of(float f) {
+    const __bf16 h = (__bf16)f;
+    uint16_t b;
+    __builtin_memcpy(&b, &h, sizeof(b));
+    return b;
+}
 __device__ inline float bf16_float(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 __device__ inline float bf16_round(float f) { return bf16_float(bf16_bits(f)); }
 
@@ -43,6 +52,11 @@ struct MlpW {
     mlp_f4 b2[4];
     mlp_f4 w3[4];      // BF16-rounded w3[16u + 4g + i]
     float b3;
+    __device__ mlp_s4 in(int t) const { return w1[t]; }
+    __device__ mlp_s4 mid(int u, int t) const { return w2t[u][t]; }
+    __device__ mlp_f4 bias1(int t) const { return b1[t]; }
+    __device__ mlp_f4 bias2(int u) const { return b2[u]; }
+    __device__ mlp_f4 out(int u) const { return w3[u]; }
 };
 
 __device__ inline void mlp_load(const float *P, MlpW &W) {
@@ -77,25 +91,29 @@ struct MlpAct {
 };
 
 // x: the B operand of layer 1 (lane supplies features 4g..4g+3 of sample r; zeros for g >= 2)
-__device__ inline void mlp_forward_tile(const MlpW &W, mlp_s4 x, MlpAct &A) {
+// W hands out the operands from where the kernel keeps them.
+template <class Weights>
+__device__ inline void mlp_forward_tile(const Weights &W, mlp_s4 x, MlpAct &A) {
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-        A.z1[t] = mfma16(W.w1[t], x, W.b1[t]);
+        A.z1[t] = mfma16(W.in(t), x, W.bias1(t));
 #pragma unroll
-        for (int i = 0; i < 4; i++) A.h1[t][i] = (short)bf16_bits(fmaxf(A.z1[t][i], 0.0f));
+        for (int i = 0; i < 4; i++) A.h1[t][i] = (short)bf16_of(fmaxf(A.z1[t][i], 0.0f));
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-        mlp_f4 acc = W.b2[u];
+        mlp_f4 acc = W.bias2(u);
 #pragma unroll
-        for (int t = 0; t < 4; t++) acc = mfma16(W.w2t[u][t], A.h1[t], acc);
+        for (int t = 0; t < 4; t++) acc = mfma16(W.mid(u, t), A.h1[t], acc);
         A.z2[u] = acc;
     }
     float p = 0.0f;
 #pragma unroll
-    for (int u = 0; u < 4; u++)
+    for (int u = 0; u < 4; u++) {
+        const mlp_f4 w3 = W.out(u);
 #pragma unroll
-        for (int i = 0; i < 4; i++) p += W.w3[u][i] * fmaxf(A.z2[u][i], 0.0f);
+        for (int i = 0; i < 4; i++) p += w3[i] * fmaxf(A.z2[u][i], 0.0f);
+    }
     p += __shfl_xor(p, 16);
     p += __shfl_xor(p, 32);
     A.z = p + W.b3;

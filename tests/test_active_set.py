@@ -118,6 +118,26 @@ def test_gpu_gradient_matches_oracle(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 15, 65, 32768, 32785, 70001])
+def test_gpu_gradient_tiles_and_rows(n):
+    """Less than a tile, a workgroup with idle wavefronts, one tile for every
+    wavefront of the largest grid, and several with a ragged last one: every
+    parameter within the sum of the BF16 roundings, 2^-8 of the magnitudes
+    that enter it (weights, activations and deltas, each rounded once)."""
+    import torch
+    from grappolo_amd import active_set as las
+    P = om.init(11)
+    P[om.B1:om.W2] = 0.02
+    P[om.B2:om.W3] = -0.01
+    feats, labels, X, y = _dev_batch(n, 4)
+    loss, g = las.grad_dev(torch.from_numpy(P).cuda(), feats, labels, pos_weight=4.0)
+    g = g.cpu().numpy().astype(np.float64)
+    lr, gr = om.loss_grad(P, X, y, 4.0, rounding=True)
+    assert loss == pytest.approx(lr, rel=1e-4)
+    assert np.linalg.norm(g - gr) <= 3 * 2.0 ** -8 * np.linalg.norm(gr)
+
+
+@pytest.mark.gpu
 def test_gpu_gradient_is_deterministic():
     import torch
     from grappolo_amd import active_set as las
