@@ -176,7 +176,14 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
     const i64 nv = g.nv;
     if (nv == 0) return -1;
     launch_fill_i32(colors, nv, -1, s_);
-    const int pnb = (int)std::min<i64>({(i64)jp_persistent_blocks(), (i64)tune_.jp_blocks,
+    // The shapes left at their defaults follow the graph.  Workgroups of the
+    // persistent rounds: 64 to 128 (RMAT, 4.2M vertices: 25.1 ms with 64, 23.6
+    // with 128, 24.3 with 256; 250,000: 4.78, 4.82, 4.79).  The core's degree:
+    // kJpCoreDeg.
+    const i64 jp_blocks = tune_.jp_blocks != kJpBlocks ? tune_.jp_blocks
+                                                       : std::min<i64>(2 * kJpBlocks, std::max<i64>(kJpBlocks, nv / 4096));
+    const i64 core_deg = tune_.core_min_deg != kJpCoreMinDeg ? tune_.core_min_deg : kJpCoreDeg;
+    const int pnb = (int)std::min<i64>({(i64)jp_persistent_blocks(), jp_blocks,
                                          std::max<i64>(4, nv / 2048)});
     DBuf<i64> ring(10, s_);
     DBuf<unsigned> bar(kJpBarrierWords, s_);
@@ -191,8 +198,8 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
     cur.dep = next.dep = dep.p;
 
     // the core: every vertex of a small graph; on a larger one the vertices
-    // of the largest degrees, at most kJpCoreMax, when they reach the tuned
-    // core degree (kJpCoreMinDeg by default)
+    // of the largest degrees, at most kJpCoreMax, when they reach the core
+    // degree
     u64 dcore = kJpNoCore;
     i64 K = 0;
     if (nv <= kJpCoreMax) {
@@ -211,7 +218,7 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
             if (above + (i64)h[b] > kJpCoreMax) break;
             above += (i64)h[b];
             const i64 lo = jp_bucket_lo(b);
-            if (lo >= tune_.core_min_deg && lo < (i64(1) << 23) && above > 0) {
+            if (lo >= core_deg && lo < (i64(1) << 23) && above > 0) {
                 dcore = (u64)lo;
                 K = above;
             }

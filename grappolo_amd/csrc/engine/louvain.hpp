@@ -111,10 +111,12 @@ BinConfig &current_bins();
 // None of them changes a result: they choose grids and which vertices the
 // coloring's core pass takes.
 struct Tuning {
-    int jp_blocks = 64;                // grid of the persistent coloring rounds (<= kJpPersistMaxBlocks)
+    int jp_blocks = kJpBlocks;         // grid of the persistent coloring rounds (<= kJpPersistMaxBlocks;
+                                       // the default: by the graph's size)
     i64 core_min_deg = kJpCoreMinDeg;  // a coloring core of a large graph starts at this degree or above
+                                       // (the default: kJpCoreDeg)
     int persist_blocks = 64;           // grid of the persistent sweep at most (<= kPersistMaxBlocks)
-    int wide_blocks = 0;               // grid of the whole-GPU sweep (0: one workgroup per CU)
+    int wide_blocks = 0;               // grid of the whole-GPU sweep at most (0: one workgroup per CU)
 };
 Tuning &current_tuning();
 bool valid_tuning(const Tuning &t);

@@ -458,3 +458,19 @@ def test_degree_sums_across_row_lengths(low):
     Co, so = oracle.run_basic(g)
     np.testing.assert_array_equal(C, Co)
     assert st["final_modularity"] == so["final_modularity"]
+
+
+@pytest.mark.parametrize("which", ["full_core", "few_core", "lfr", "rmat15"])
+def test_coloring_core_of_light_vertices(which):
+    """Cores that start at degree 64: more vertices of such degrees than the
+    core holds (rounds of thousands in one workgroup, the rest by frontier
+    rounds), a few of them, and skewed graphs just above 16384 vertices."""
+    from grappolo_amd.graph import gen_lfr, gen_planted, gen_rmat
+    g = {"full_core": lambda: gen_planted(20000, 8, 100, 0.4, seed=3),
+         "few_core": lambda: gen_planted(17000, 8, 45, 0.3, seed=4),
+         "lfr": lambda: gen_lfr(16385, seed=5),
+         "rmat15": lambda: gen_rmat(15, seed=6)}[which]()
+    colors, mc = engine.algoDistanceOneVertexColoringOpt(g)
+    ref, rmc, _ = oracle.color_jp(g)
+    assert mc == rmc
+    np.testing.assert_array_equal(colors, ref)
