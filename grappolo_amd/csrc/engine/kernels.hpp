@@ -243,9 +243,13 @@ void launch_jp_degree_hist(const DevGraph &g, unsigned long long *hist, hipStrea
 // their index (flags, pos: nv scratch)
 void launch_jp_core_list(const DevGraph &g, u64 dcore, i64 *flags, i64 *pos, i64 *hlist, int32_t *cnt,
                          hipStream_t s);
-// sizes[q] = core neighbours of core vertex q (q < K), sizes[K] = 0
+// sizes[q] = units of the list of core vertex q (q < K), sizes[K] = 0; loff[q]:
+// the units before it
 void launch_jp_core_sizes(const int32_t *core_cnt, i64 K, i64 *sizes, hipStream_t s);
-// ladj[loff[q] ..): the core indices of core vertex q's higher core
+// ladj entries that lists of that many units need (16-byte aligned): the core's
+// workgroup loads the entries of its first turn before it knows a list's length
+i64 jp_core_list_entries(i64 units);
+// ladj: the lists, a head and the core indices of core vertex q's higher core
 // neighbours, then of its lower ones (codes of the count)
 void launch_jp_core_fill(const DevGraph &g, const uint8_t *code, const int32_t *cnt, const i64 *hlist, i64 K,
                          const i64 *loff, const int32_t *core_cnt, uint16_t *ladj, hipStream_t s);

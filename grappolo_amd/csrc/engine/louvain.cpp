@@ -247,7 +247,7 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
     // count), per vertex 20 (offsets, priority, count); the tail's first-fit
     // over at most kJpTail vertices is left out
     Profiler::get().end(K_COLOR, 30.0 * g.nnz + 20.0 * nv, s_);
-    i64 core_entries = 0;
+    i64 core_units = 0;
     if (K > 0) {
         DBuf<i64> sizes(K + 1, s_);  // (the giant lists hold the count's frontier)
         launch_jp_core_sizes(core_cnt.p, K, sizes.p, s_);
@@ -256,12 +256,12 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
     {
         Readback rb(s_);
         rb.add(hc, cur.counts, sizeof(hc));
-        if (K > 0) rb.add(&core_entries, loff.p + K, sizeof(i64));
+        if (K > 0) rb.add(&core_units, loff.p + K, sizeof(i64));
         rb.run();
     }
     i64 colored = 0;
     if (K > 0) {
-        DBuf<uint16_t> ladj(std::max<i64>(core_entries, 1), s_);
+        DBuf<uint16_t> ladj(jp_core_list_entries(core_units), s_);
         Profiler::get().begin(K_COLOR, s_);
         launch_jp_core_fill(g, code.p, cnt.p, hlist.p, K, loff.p, core_cnt.p, ladj.p, s_);
         // a core that is the whole graph stops where the tail starts
