@@ -19,7 +19,7 @@ enum KClass {
     K_PERSIST = 13,  // one persistent launch per colored iteration of a small graph
     K_COLOR_TAIL = 14,  // sequential first-fit of the vertices JP rounds left
     K_SWEEP_GIANT = 15,  // sweep of degree bin 9 (giant vertices, several workgroups each)
-    K_WIDE = 16,         // one whole-GPU persistent launch per colored iteration of a large graph
+    K_WIDE = 16,         // one whole-GPU persistent launch per colored iteration of a graph above kPersistMaxNV
     K_NUM = 17
 };
 inline int sweep_class(int bin) { return bin <= 8 ? K_SWEEP_B1 + bin - 1 : K_SWEEP_GIANT; }
