@@ -2648,12 +2648,17 @@ __global__ __launch_bounds__(kBlock) void k_tail_prep(const i64 *off, const i64 
 // neither base[t] nor an earlier tail neighbour holds once all of those have
 // theirs -- the sequential result, in as many rounds as the longest chain of
 // earlier neighbours (a dozen in sparse tails, where one vertex after the
-// other took 0.55 us each).  A round: the ready vertices are listed, a
+// other took 0.55 us each).  A round takes 2.6 us, so the rounds go on while
+// they colour kTailPace vertices each on average; a tail close to a clique is
+// finished one vertex after the other (1024 of them: 0.6 ms, 2.7 in rounds).
+// A round: the ready vertices are listed, a
 // wavefront each gathers the neighbours' colours, two workgroup barriers.  In
 // LDS: the bit rows without the words no earlier vertex can be in, word-major
 // so that the threads' checks do not conflict, and the first kTailWords words
 // of the base rows (the rest is read from HBM when those are all taken).
 constexpr int kTailWords = 16;
+constexpr int kTailPace = 5, kTailTrial = 8;  // judged from this round on
+constexpr int kTailBatch = 8;                 // base rows fetched together
 constexpr int kTailRows = (int)(kJpTail / 64);
 // word w of row t (t >= 64 w)
 __device__ inline int tail_word(int w, int t) { return w * (int)kJpTail - 32 * w * (w - 1) + t - 64 * w; }
@@ -2679,7 +2684,9 @@ __global__ __launch_bounds__(kTailBlock) void k_tail_rounds(const i64 *list, int
     __syncthreads();
     bool todo = t < n;
     int at = 0;  // the first word of the row with a neighbour not yet coloured
-    for (int left = n, round = 0; left > 0; round = round == 2 ? 0 : round + 1) {
+    int left = n;
+    for (int round = 0, rounds = 0; left > 0; round = round == 2 ? 0 : round + 1, rounds++) {
+        if (rounds >= kTailTrial && n - left < kTailPace * rounds) break;
         bool ready = todo;
         if (todo)
             for (; at <= t / 64; at++)
@@ -2739,6 +2746,43 @@ __global__ __launch_bounds__(kTailBlock) void k_tail_rounds(const i64 *list, int
         }
         left -= nr;
         __syncthreads();
+    }
+    if (left > 0) {
+        // the rest one after the other: vertex i's forbidden colours are base[i]
+        // plus those of the set bits of row i, each brought by its own thread
+        static_assert(kTailBatch * FW <= (kTailBlock / kWave) * FW && FW % kWave == 0, "the rows fit s_forb");
+        int mine = t < n ? s_color[t] : 0;  // (of an uncoloured vertex: set before it is used)
+        for (int i0 = 0; i0 < n; i0 += kTailBatch) {
+            __syncthreads();  // the previous batch is done with s_forb
+            for (int x = t; x < kTailBatch * FW; x += kTailBlock)
+                s_forb[x / FW][x % FW] = i0 + x / FW < n ? base[(i64)(i0 + x / FW) * FW + x % FW] : 0u;
+            __syncthreads();
+            for (int i = i0; i < i0 + kTailBatch && i < n; i++) {
+                if ((s_done[i >> 6] >> (i & 63)) & 1) continue;  // (s_done is settled: all threads agree)
+                uint32_t *forb = s_forb[i - i0];
+                if (t < i && ((s_adj[tail_word(t >> 6, i)] >> lane) & 1)) atomicOr(&forb[mine >> 5], 1u << (mine & 31));
+                __syncthreads();
+                // every wavefront finds the first free colour by itself
+                int c = kMaxColors;
+                for (int x = lane; x < FW; x += kWave) {
+                    const uint32_t f = forb[x];
+                    if (f != 0xFFFFFFFFu && c == kMaxColors) c = 32 * x + __ffs((int)~f) - 1;
+                }
+#pragma unroll
+                for (int o = kWave / 2; o > 0; o >>= 1) {
+                    const int x = __shfl_xor(c, o);
+                    c = x < c ? x : c;
+                }
+                if (c >= kMaxColors) {
+                    if (t == 0) atomicOr(err, 1);
+                    c = 0;
+                }
+                if (t == i) {
+                    mine = c;
+                    s_color[t] = (uint16_t)c;
+                }
+            }
+        }
     }
     if (t < n && list[t] >= 0 && list[t] < nv) colors[list[t]] = s_color[t];
 }
