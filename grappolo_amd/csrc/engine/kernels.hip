@@ -2648,9 +2648,10 @@ __global__ __launch_bounds__(kBlock) void k_tail_prep(const i64 *off, const i64 
 // neither base[t] nor an earlier tail neighbour holds once all of those have
 // theirs -- the sequential result, in as many rounds as the longest chain of
 // earlier neighbours (a dozen in sparse tails, where one vertex after the
-// other took 0.55 us each).  A round takes 2.6 us, so the rounds go on while
-// they colour kTailPace vertices each on average; a tail close to a clique is
-// finished one vertex after the other (1024 of them: 0.6 ms, 2.7 in rounds).
+// other took 0.55 us each).  A round takes 2.6 to 3.7 us, so the rounds go on
+// while they colour kTailPace vertices each on average; a tail close to a clique
+// is finished one vertex after the other (the four tails of an LFR graph of 4.2
+// million vertices, two of them dense: 2.3 ms a run, 8.3 in rounds alone).
 // A round: the ready vertices are listed, a
 // wavefront each gathers the neighbours' colours, two workgroup barriers.  In
 // LDS: the bit rows without the words no earlier vertex can be in, word-major
