@@ -2964,15 +2964,57 @@ __global__ __launch_bounds__(kBlock) void k_jp_finish(const int32_t *colors, i64
     if (threadIdx.x == 0 && s_m >= 0) atomicMax(maxc, s_m);
 }
 
-__global__ void k_color_conflicts(const i64 *off, const i64 *tails, i64 nv, const int32_t *colors,
-                                  i64 *count) {
-    i64 local = 0;
-    for (i64 v = blockIdx.x * (i64)blockDim.x + threadIdx.x; v < nv; v += (i64)gridDim.x * blockDim.x)
-        for (i64 j = off[v]; j < off[v + 1]; j++) {
-            i64 u = tails[j];
-            if (u != v && colors[u] == colors[v]) local++;
+// *count += the entries whose ends share a color, self-loops aside: G lanes per
+// row, rows of more than 64 G entries listed for k_color_conflicts_hub, a
+// workgroup each (a thread per row took a hub's entries one after the other:
+// %%HUB%%).
+__device__ inline void add_count(unsigned local, i64 *count) {
+    __shared__ unsigned s_local;
+    __syncthreads();
+    if (threadIdx.x == 0) s_local = 0;
+    __syncthreads();
+    if (local) atomicAdd(&s_local, local);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_local) atomicAdd((unsigned long long *)count, (unsigned long long)s_local);
+}
+template <int G>
+__global__ __launch_bounds__(kBlock) void k_color_conflicts(const i64 *off, const i64 *tails, i64 nv,
+                                                            const int32_t *colors, i64 *count, i64 *hubs,
+                                                            unsigned long long *nhubs) {
+    const int gl = threadIdx.x % G;
+    unsigned local = 0;
+    for (i64 v = (blockIdx.x * (i64)kBlock + threadIdx.x) / G; v < nv; v += (i64)gridDim.x * kBlock / G) {
+        const i64 beg = off[v], end = off[v + 1];
+        if (end - beg > 64 * G) {
+            if (gl == 0) hubs[atomicAdd(nhubs, 1ULL)] = v;
+            continue;
         }
-    if (local) atomicAdd((unsigned long long *)count, (unsigned long long)local);
+        const int32_t s = colors[v];
+        for (i64 j0 = beg + gl; j0 < end; j0 += 4 * G) {
+            i64 t[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) t[u] = j0 + u * G < end ? tails[j0 + u * G] : v;
+#pragma unroll
+            for (int u = 0; u < 4; u++) local += t[u] != v && colors[t[u]] == s;
+        }
+    }
+    add_count(local, count);
+}
+__global__ __launch_bounds__(kSumBlock) void k_color_conflicts_hub(const i64 *off, const i64 *tails,
+                                                                   const int32_t *colors, i64 *count,
+                                                                   const i64 *hubs,
+                                                                   const unsigned long long *nhubs) {
+    const i64 n = (i64)*nhubs;
+    for (i64 q = blockIdx.x; q < n; q += gridDim.x) {
+        const i64 v = hubs[q], end = off[v + 1];
+        const int32_t s = colors[v];
+        unsigned local = 0;
+        for (i64 j = off[v] + threadIdx.x; j < end; j += kSumBlock) {
+            const i64 t = tails[j];
+            local += t != v && colors[t] == s;
+        }
+        add_count(local, count);
+    }
 }
 
 // ------------------------------------------------------------------- renumber
@@ -3320,6 +3362,15 @@ void launch_color_major(const i64 *perm, const int32_t *colors, i64 n, int ncol,
     k_slice_starts<<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(keys.p, n, ncol, cstart);
     GLV_LAUNCH_CHECK();
 }
+// f(lanes per row) for a pass over the rows: about half the mean degree
+template <class F>
+static void with_row_lanes(const DevGraph &g, F f) {
+    const i64 mean = g.nnz / g.nv;
+    if (mean <= 8) f(std::integral_constant<int, 4>());
+    else if (mean <= 16) f(std::integral_constant<int, 8>());
+    else if (mean <= 64) f(std::integral_constant<int, 16>());
+    else f(std::integral_constant<int, 64>());
+}
 void launch_slices(const uint32_t *sorted_keys, const i64 *perm, const i64 *off, i64 n, i64 nkeys,
                    i64 *start, i64 *pnnz, hipStream_t s) {
     if (n <= 0) return;
@@ -3666,7 +3717,16 @@ void launch_jp_finish(int32_t *state, i64 nv, int32_t *maxc, hipStream_t s) {
 }
 void launch_color_conflicts(const DevGraph &g, const int32_t *colors, i64 *count, hipStream_t s) {
     if (g.nv <= 0) return;
-    k_color_conflicts<<<grid_for(g.nv, kBlock, 8192), kBlock, 0, s>>>(g.off, g.tails, g.nv, colors, count);
+    DBuf<i64> hubs(g.nv, s);
+    DBuf<unsigned long long> nhubs(1, s);
+    launch_fill_i64((i64 *)nhubs.p, 1, 0, s);
+    with_row_lanes(g, [&](auto lanes) {
+        constexpr int G = decltype(lanes)::value;
+        k_color_conflicts<G><<<grid_for(g.nv * G, kBlock, 8192), kBlock, 0, s>>>(g.off, g.tails, g.nv, colors, count,
+                                                                                 hubs.p, nhubs.p);
+    });
+    GLV_LAUNCH_CHECK();
+    k_color_conflicts_hub<<<1024, kSumBlock, 0, s>>>(g.off, g.tails, colors, count, hubs.p, nhubs.p);
     GLV_LAUNCH_CHECK();
 }
 
@@ -3778,17 +3838,11 @@ static void row_sums(const DevGraph &g, const int32_t *C, const int32_t *lab, do
     DBuf<i64> hubs(g.nv, s);
     DBuf<unsigned long long> nhubs(1, s);
     launch_fill_i64((i64 *)nhubs.p, 1, 0, s);
-    // lanes per row: about half the mean degree
-    const i64 mean = g.nnz / g.nv;
-    auto go = [&](auto lanes) {
+    with_row_lanes(g, [&](auto lanes) {
         constexpr int G = decltype(lanes)::value;
         k_row_sums<G, LAB><<<grid_for(g.nv * G, kBlock, 8192), kBlock, 0, s>>>(g.off, g.tails, g.w, C, lab, g.nv, rk,
                                                                                re, hubs.p, nhubs.p);
-    };
-    if (mean <= 8) go(std::integral_constant<int, 4>());
-    else if (mean <= 16) go(std::integral_constant<int, 8>());
-    else if (mean <= 64) go(std::integral_constant<int, 16>());
-    else go(std::integral_constant<int, 64>());
+    });
     GLV_LAUNCH_CHECK();
     k_row_sums_hub<LAB><<<1024, kSumBlock, 0, s>>>(g.off, g.tails, g.w, C, lab, rk, re, hubs.p, nhubs.p);
     GLV_LAUNCH_CHECK();

@@ -387,11 +387,15 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
     return fetch(maxc.p);
 }
 
-i64 Engine::count_conflicts(const DevGraph &g, const int32_t *colors) {
+i64 Engine::conflicting_entries(const DevGraph &g, const int32_t *colors) {
     DBuf<i64> c(1, s_);
     launch_fill_i64(c.p, 1, 0, s_);
     launch_color_conflicts(g, colors, c.p, s_);
-    return fetch(c.p) / 2;
+    return fetch(c.p);
+}
+i64 Engine::count_conflicts(const DevGraph &g, const int32_t *colors) { return conflicting_entries(g, colors) / 2; }
+bool Engine::proper_coloring(const DevGraph &g, const int32_t *colors) {
+    return colors && conflicting_entries(g, colors) == 0;
 }
 
 // --------------------------------------------------------------- modularity
@@ -431,7 +435,7 @@ static i64 mod_part_count(const PhaseSetup &P) {
 // With a learned active set (las), see LasParams.
 double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, int ncol, double Lower,
                              double thresh, int *iters, std::vector<double> *trace, LasParams *las,
-                             int phase_index, bool valid_colors) {
+                             int phase_index, Proper proper) {
     const i64 nv = g.nv;
     PhaseSetup P;
     setup(g, colors, ncol, P);
@@ -553,6 +557,8 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     DBuf<uint32_t> wtpos;
     DBuf<i64> wtoff(use_wide ? nv + 1 : 0, s_);
     bool labels32 = false;
+    const bool valid_colors =
+        proper == Proper::unknown ? (use_wide || !persistent) && proper_coloring(g, colors) : proper == Proper::yes;
     if (use_wide) {
         launch_narrow_ids(C, nv, wc.p, s_);
         group_entries_by_tail(g, wlab.p, wtpos, wtoff.p, s_);
@@ -1163,7 +1169,8 @@ void Engine::run_colored(const DevGraph &g0, i64 *C_orig, const RunParams &p, Ru
         const i64 swept0 = p.las ? p.las->swept_entries : 0;
         if (!nonColor) {
             currMod = colored_phase(*G, Cbuf.p, colors.p, nColors, currMod, p.C_threshold, &tmpItr,
-                                    &r.trace, p.las, phase - 1, fresh_colors && p.coloring != 3);
+                                    &r.trace, p.las, phase - 1,
+                                    fresh_colors && p.coloring != 3 ? Proper::yes : Proper::no);
             rec.colored = 1;
             rec.ncolors = nColors;
             r.edges_visited_mod += (i64)tmpItr * G->nnz;

@@ -139,16 +139,22 @@ public:
     // the coloring step of runMultiPhaseColoring.cpp:68-87 for p.coloring;
     // returns nColors (largest color + 1)
     int color_for_run(const DevGraph &g, int32_t *colors, const RunParams &p);
+    // edges whose ends share a color
     i64 count_conflicts(const DevGraph &g, const int32_t *colors);
+    // no entry's ends do
+    bool proper_coloring(const DevGraph &g, const int32_t *colors);
 
     // algoLouvainWithDistOneColoring: C (device, nv) receives the labels.
-    // valid_colors: the classes are independent sets of g (a fresh distance-1
-    // coloring), so a color step's moves change the internal weight by exactly
-    // the movers' 2 (e_vt - e_vs) and iterations after the first need no full
-    // modularity pass
+    // proper: whether the classes are independent sets of g (a fresh distance-1
+    // coloring).  A color step's moves then change the internal weight by exactly
+    // the movers' 2 (e_vt - e_vs), iterations after the first need no full
+    // modularity pass, and the whole-GPU sweep needs one grid barrier per step
+    // instead of two.  Unknown (a caller's colors): found out by one pass over
+    // the entries where it matters
+    enum class Proper { unknown, yes, no };
     double colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, int ncol, double Lower,
                          double thresh, int *iters, std::vector<double> *trace = nullptr,
-                         LasParams *las = nullptr, int phase_index = 0, bool valid_colors = false);
+                         LasParams *las = nullptr, int phase_index = 0, Proper proper = Proper::unknown);
     // parallelLouvianMethod(NoMap): C receives pastCommAss
     double plain_phase(const DevGraph &g, i64 *C, double Lower, double thresh, bool nomap,
                        int *iters, std::vector<double> *trace = nullptr);
@@ -180,6 +186,7 @@ private:
     // small pinned-free scratch for scalars copied back to the host
     template <class T>
     T fetch(const T *dptr);
+    i64 conflicting_entries(const DevGraph &g, const int32_t *colors);
     double colored_modularity(const DevGraph &g, const PhaseSetup &P, const i64 *C,
                               double *part, double *res, double *exx = nullptr);
 };

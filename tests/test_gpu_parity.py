@@ -474,3 +474,25 @@ def test_coloring_core_of_light_vertices(which):
     ref, rmc, _ = oracle.color_jp(g)
     assert mc == rmc
     np.testing.assert_array_equal(colors, ref)
+
+
+@pytest.mark.parametrize("mean", [2, 9, 20, 120])
+def test_conflicts_counted_over_row_lengths(mean):
+    """Edges inside a color class, counted 4 to 64 lanes a row and by a
+    workgroup for rows beyond 64 entries a lane: rows at those bounds,
+    self-loops (no conflict), few and many colors, against a count in numpy."""
+    import torch
+    nv = 4001
+    rng = np.random.default_rng(mean)
+    m = nv * mean // 2
+    loops = np.arange(5, nv, 97)
+    pairs = [np.stack([rng.integers(20, nv - 30, m), rng.integers(20, nv - 30, m)], 1), np.stack([loops, loops], 1)]
+    for h, d in enumerate([255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 3900]):
+        pairs.append(np.stack([np.full(d, h), 20 + rng.choice(nv - 50, d, replace=False)], 1))
+    g = Graph.from_pairs(nv, np.unique(np.sort(np.concatenate(pairs), 1), axis=0))
+    rows = np.repeat(np.arange(nv), g.degrees())
+    dg = engine.DeviceGraph(g)
+    for k in (1, 3, 400):
+        colors = rng.integers(0, k, nv).astype(np.int32)
+        exp = np.count_nonzero((rows < g.tails) & (colors[rows] == colors[g.tails]))
+        assert engine.count_conflicts_dev(dg, torch.from_numpy(colors).cuda()) == exp

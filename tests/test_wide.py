@@ -119,6 +119,38 @@ def test_phase_on_both_sides_of_the_dense_limit(nv, valid):
     np.testing.assert_array_equal(C, Co)
 
 
+@pytest.mark.parametrize("conflicts", [0, 1])
+def test_phase_with_a_callers_colors(conflicts):
+    """The stage entry point finds out whether the colors it is given are
+    proper: then one full modularity pass serves the phase, with a single edge
+    inside a class (of the hub, whose row a workgroup scans) every iteration
+    takes one; labels, iterations and modularity equal the oracle's either way."""
+    from grappolo_amd import engine
+    from grappolo_amd.graph import Graph, gen_planted
+    nv = 20000
+    core = gen_planted(nv, 20, 12, 0.25, seed=1)
+    rows = np.repeat(np.arange(nv), core.degrees())
+    keep = (rows < core.tails) & (rows > 0)
+    hub = np.stack([np.zeros(6000, np.int64), np.arange(1, 6001)], 1)
+    g = Graph.from_pairs(nv, np.concatenate([hub, np.stack([rows[keep], core.tails[keep]], 1)]))
+    colors, mc = oracle.color_greedy(g)
+    colors = colors.astype(np.int32)
+    if conflicts:  # neighbour 6000 of the hub takes the hub's color, which none of its other neighbours has
+        mc += 1
+        colors[[0, 6000]] = mc
+    engine.profile_reset()
+    engine.profile_enable(True)
+    try:
+        q, C, it = engine.algoLouvainWithDistOneColoring(g, colors, mc + 1, -1.0, 1e-6)
+    finally:
+        engine.profile_enable(False)
+    assert it > 2
+    assert engine.profile_read()["modularity"][2] == (it if conflicts else 1)
+    qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+    assert it == ito and q == qo
+    np.testing.assert_array_equal(C, Co)
+
+
 @pytest.mark.parametrize("stage", ["run", "phase"])
 def test_degrees_at_the_item_bounds(stage):
     """Vertices whose entries sit at the bounds of the sweep's work items
@@ -126,7 +158,8 @@ def test_degrees_at_the_item_bounds(stage):
     8192, one and several chunks of 4096, a table round past each) on a
     planted background: the run's labels (labels pushed in the step; the
     giants merged once few communities are left) and the stage entry point's
-    (pushed after the step, since it takes any colors) equal the oracle's."""
+    (with one edge inside a class, so that labels are pushed after the step)
+    equal the oracle's."""
     import torch
     from grappolo_amd import engine
     from grappolo_amd.graph import Graph, gen_planted
@@ -151,6 +184,8 @@ def test_degrees_at_the_item_bounds(stage):
         np.testing.assert_array_equal(C.cpu().numpy(), Co)
     else:
         colors, mc = oracle.color_greedy(g)
+        v = int(g.edgeListPtrs[nh])  # the first planted vertex takes its first neighbour's color
+        colors[nh] = colors[g.tails[v]]
         q, C, it = engine.algoLouvainWithDistOneColoring(g, colors, mc + 1, -1.0, 1e-6)
         qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
         assert it == ito and q == qo
