@@ -452,9 +452,16 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         color_nonempty[c] = size > 0;
         max_class = std::max(max_class, size);
     }
-    int nonempty = 0;
-    for (int c = 0; c < ncol; c++) nonempty += color_nonempty[c];
+    int nonempty = 0, bins = 0;  // classes, and their non-empty bins in all
+    for (int c = 0; c < ncol; c++) {
+        nonempty += color_nonempty[c];
+        for (int b = 1; b < kNumBins; b++) bins += P.hi(b, c) > P.lo(b, c);
+    }
     const i64 per_class = (nv + std::max(nonempty, 1) - 1) / std::max(nonempty, 1);
+    auto classes_proper = [&] {
+        if (proper == Proper::unknown) proper = proper_coloring(g, colors) ? Proper::yes : Proper::no;
+        return proper == Proper::yes;
+    };
     // graphs above the dense sweep's vertices, or whose classes are large: the
     // whole-GPU persistent sweep (wide.hpp), plain form only.  Classes of more than kWideMaxPerColor
     // vertices on average fill the GPU with per-color launches of the binned
@@ -462,18 +469,40 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     // and of the hash form of the persistent sweep: a 250,007-vertex RMAT run
     // went from 363 to 103 ms (its per-color launches took 13 ms per
     // iteration, most of it one HBM-table launch per class), a 62,103-vertex
-    // coarse phase of 69 colors from 45.2 to 14.9 ms.  Dense phases (<= 15,360
-    // vertices) with classes of kWideDensePerColor vertices or more take it too
-    // (the dense sweep gives every vertex a workgroup of its own: a phase of
-    // 15,000 vertices and 9 colors 49.9 -> 8.0 ms, of 14,588 and 83 41.5 -> 23.2,
-    // of 1392 and 16 2.6 -> 2.4); with smaller classes the dense sweep's shorter
-    // steps win (1682 vertices, 50 colors: 5.9 ms against 7.1).
+    // coarse phase of 69 colors from 45.2 to 14.9 ms.
+    //
+    // Not so where the launches are few and full (wide.hpp, kWideLight*): no
+    // vertex above 256 entries, and a class takes about two launches or is
+    // large.  They need no item plan and no entry positions, and a class takes
+    // them 10 us against a color step's 13.  Per-color launches / this sweep, ms
+    // per phase: path of 200,000 0.4 / 0.9, grid of 400 x 400 1.4 / 2.4, of 700 x
+    // 700 2.1 / 3.4, planted 65,536 of degree 128 2.5 / 3.6, 200,000 of 128 4.8 /
+    // 6.3 and of 40 8.3 / 9.7, 500,000 of 32 14.0 / 17.1, 260,000 of 24 in 17
+    // classes 14.3 / 16.3.  On the other side: planted 65,536 of degree 16
+    // (105,000 entries and 3.1 launches a class) 5.4 / 4.9, 20,000 of degree 8 2.6
+    // / 2.1; a million of degree 100 26.3 / 21.7 (the gathered labels outgrow an
+    // XCD's L2).
+    //
+    // Dense phases (<= 15,360 vertices) with classes of kWideDensePerColor
+    // vertices or more take it too (the dense sweep gives every vertex a
+    // workgroup of its own: a phase of 15,000 vertices and 9 colors 49.9 -> 8.0
+    // ms, of 14,588 and 83 41.5 -> 23.2, of 1392 and 16 2.6 -> 2.4); with smaller
+    // classes the dense sweep's shorter steps win (1682 vertices, 50 colors: 5.9
+    // ms against 7.1), and up to twice that size when classes hold edges, which
+    // costs a second barrier per step (1392 vertices and 17 such classes: 2.9
+    // against 3.9 ms, 1682 and 17: 1.7 against 2.3; 1841 and 11: 2.4 against 1.6).
     const bool las_mode = las && !(las->mode == 2 && nv <= kDenseMaxNV) && las->mode != 0;
     int wblocks = 0;
-    if (!las_mode && (nv > kDenseMaxNV || per_class >= kWideDensePerColor) && nonempty > 0 &&
-        nv / nonempty <= kWideMaxPerColor && wide_enabled()) {
-        wblocks = wide_grid(g.nnz / nonempty);
-        if (tune_.wide_blocks > 0) wblocks = std::min(wblocks, tune_.wide_blocks);
+    if (!las_mode && nonempty > 0 && nv / nonempty <= kWideMaxPerColor && wide_enabled()) {
+        const bool light = P.bin_hi(kNumBins - 1) == P.bin_lo(7) && per_class > kPersistMaxPerColor &&
+                           nv <= kWideLightNV &&
+                           (bins <= kWideLightLaunches * nonempty || g.nnz / nonempty >= kWideLightEntries);
+        if (nv > kDenseMaxNV ? !light
+                             : per_class >= kWideDensePerColor &&
+                                   (per_class >= 2 * kWideDensePerColor || classes_proper())) {
+            wblocks = wide_grid(g.nnz / nonempty);
+            if (tune_.wide_blocks > 0) wblocks = std::min(wblocks, tune_.wide_blocks);
+        }
     }
     // coarse graphs (small, or many small color classes): one persistent
     // launch per iteration (all colors + modularity), grid sized to the color
@@ -557,8 +586,9 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     DBuf<uint32_t> wtpos;
     DBuf<i64> wtoff(use_wide ? nv + 1 : 0, s_);
     bool labels32 = false;
-    const bool valid_colors =
-        proper == Proper::unknown ? (use_wide || !persistent) && proper_coloring(g, colors) : proper == Proper::yes;
+    // (the launches take a caller's colors as they come: a full modularity pass
+    // per iteration costs them less than the movers' sums after every class)
+    const bool valid_colors = use_wide ? classes_proper() : proper == Proper::yes;
     if (use_wide) {
         launch_narrow_ids(C, nv, wc.p, s_);
         group_entries_by_tail(g, wlab.p, wtpos, wtoff.p, s_);
@@ -1170,7 +1200,9 @@ void Engine::run_colored(const DevGraph &g0, i64 *C_orig, const RunParams &p, Ru
         if (!nonColor) {
             currMod = colored_phase(*G, Cbuf.p, colors.p, nColors, currMod, p.C_threshold, &tmpItr,
                                     &r.trace, p.las, phase - 1,
-                                    fresh_colors && p.coloring != 3 ? Proper::yes : Proper::no);
+                                    !fresh_colors       ? Proper::no
+                                    : p.coloring == 3 ? Proper::unknown  // (incomplete, or not)
+                                                      : Proper::yes);
             rec.colored = 1;
             rec.ncolors = nColors;
             r.edges_visited_mod += (i64)tmpItr * G->nnz;

@@ -71,6 +71,13 @@ constexpr i64 kWideMaxPerColor = 100000;
 // vertices per color class on (the mean).
 constexpr i64 kWideDensePerColor = 64;
 
+// Phases without a vertex above 256 entries keep the per-color launches up to
+// kWideLightNV vertices (64-bit labels within an XCD's 4 MB L2) when a class
+// takes kWideLightLaunches of them on average or holds kWideLightEntries entries
+// (measured where the choice is made, Engine::colored_phase).
+constexpr i64 kWideLightNV = 524288, kWideLightEntries = 250000;
+constexpr double kWideLightLaunches = 2.2;
+
 // Relative costs of workgroup items (microseconds, measured order of
 // magnitude): a heavy vertex kWCostHeavy plus three per 1024 entries.
 constexpr double kWCostHeavy = 10.0, kWCostChunk = 10.0, kWCostPart = 10.0;

@@ -151,6 +151,52 @@ def test_phase_with_a_callers_colors(conflicts):
     np.testing.assert_array_equal(C, Co)
 
 
+@pytest.mark.parametrize("kind,route", [("ring", "launches"), ("ring_of_257", "wide"), ("planted", "wide"),
+                                        ("proper_100", "wide"), ("edges_inside_100", "dense"),
+                                        ("edges_inside_128", "wide")])
+def test_route_of_a_phase(kind, route):
+    """Per-color launches keep the phases above the dense limit whose classes
+    take a launch or two each and hold no vertex above 256 entries; the dense
+    sweep keeps classes of fewer than 64 vertices, of fewer than 128 when they
+    hold edges.  The profile tells the routes apart (the whole-GPU sweep takes a
+    modularity pass, the dense one none); all equal the oracle's color steps."""
+    from grappolo_amd import engine
+    from grappolo_amd.graph import Graph, gen_planted
+    if kind.startswith("ring"):
+        nv = 20000
+        i = np.arange(nv)
+        pairs = [np.stack([i, (i + s) % nv], 1) for s in range(1, 21)]
+        if kind != "ring":  # one vertex of 40 + 217 entries
+            pairs.append(np.stack([np.zeros(217, np.int64), 100 + 7 * np.arange(217)], 1))
+        g = Graph.from_pairs(nv, np.concatenate(pairs))
+        assert g.degrees().max() == (40 if kind == "ring" else 257)
+    else:
+        g = gen_planted(20000 if kind == "planted" else 1600, 16, 8, 0.25, seed=2)
+    nv = g.numVertices
+    if kind.startswith("edges_inside"):
+        classes = nv // int(kind[-3:])
+        colors, mc = (np.arange(nv) * 7 % classes).astype(np.int32), classes - 1
+    elif kind == "proper_100":  # greedy colors, the largest classes split
+        colors, _ = oracle.color_greedy(g)
+        colors = np.unique(colors * 2 + (np.arange(nv) % 2), return_inverse=True)[1].astype(np.int32)
+        mc = int(colors.max())
+        assert 64 <= nv / (mc + 1) < 128
+    else:
+        colors, mc = oracle.color_greedy(g)
+    engine.profile_reset()
+    engine.profile_enable(True)
+    try:
+        q, C, it = engine.algoLouvainWithDistOneColoring(g, colors, mc + 1, -1.0, 1e-6)
+    finally:
+        engine.profile_enable(False)
+    prof = engine.profile_read()
+    persistent, passes = prof["sweep_persistent_iteration"][2], prof["modularity"][2]
+    assert (persistent, passes > 0) == {"launches": (0, True), "wide": (it, True), "dense": (it, False)}[route]
+    qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+    assert it == ito and q == qo
+    np.testing.assert_array_equal(C, Co)
+
+
 @pytest.mark.parametrize("stage", ["run", "phase"])
 def test_degrees_at_the_item_bounds(stage):
     """Vertices whose entries sit at the bounds of the sweep's work items
