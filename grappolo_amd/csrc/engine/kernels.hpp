@@ -73,9 +73,9 @@ void launch_bin_keys(const i64 *off, i64 nv, const int32_t *colors, int ncol, ui
 void launch_slices(const uint32_t *sorted_keys, const i64 *perm, const i64 *off, i64 n, i64 nkeys,
                    i64 *start, i64 *pnnz, hipStream_t s);
 // k = sums of the rows: of at most `cut` entries (all rows), mid (listed, up to
-// kBinMaxDeg[7] entries), big (listed, longer)
-void launch_degree(const DevGraph &g, i64 cut, const i64 *mid, i64 nmid, const i64 *big, i64 nbig, double *k,
-                   hipStream_t s);
+// kBinMaxDeg[6] entries), heavy (listed, up to kBinMaxDeg[7]), big (listed, longer)
+void launch_degree(const DevGraph &g, i64 cut, const i64 *mid, i64 nmid, const i64 *heavy, i64 nheavy,
+                   const i64 *big, i64 nbig, double *k, hipStream_t s);
 void launch_init_comm(const double *k, i64 nv, double *a, i64 *n, hipStream_t s);
 void launch_comm_from_labels(const i64 *C, const double *k, i64 nv, double *a, i64 *n,
                              hipStream_t s);

@@ -95,15 +95,14 @@ void Engine::setup(const DevGraph &g, const int32_t *colors, int ncol, PhaseSetu
         }
     }
     // degrees and 1/(2m)
-    const i64 big_lo = P.bin_lo(8), big_hi = P.bin_hi(9);
-    const i64 mid_lo = P.bin_lo(6);
-    launch_degree(g, bins_.max_deg[5], P.perm.p + mid_lo, big_lo - mid_lo, P.perm.p + big_lo, big_hi - big_lo, P.k.p,
-                  s_);
+    const i64 *mid = P.perm.p + P.bin_lo(6), *heavy = P.perm.p + P.bin_lo(7), *big = P.perm.p + P.bin_lo(8);
+    launch_degree(g, bins_.max_deg[5], mid, heavy - mid, heavy, big - heavy, big, P.bin_hi(9) - P.bin_lo(8), P.k.p, s_);
     DBuf<double> part(kRedBlocks, s_), res(1, s_);
     launch_sum(P.k.p, nv, part.p, res.p, s_);
     P.total_weight = fetch(res.p);
     P.constant = (double)1 / P.total_weight;
     P.maxdeg_global = 0;
+    const i64 big_lo = P.bin_lo(8);
     if (P.bin_hi(8) > big_lo) {
         DBuf<i64> md(1, s_);
         launch_fill_i64(md.p, 1, 0, s_);

@@ -496,3 +496,21 @@ def test_conflicts_counted_over_row_lengths(mean):
         colors = rng.integers(0, k, nv).astype(np.int32)
         exp = np.count_nonzero((rows < g.tails) & (colors[rows] == colors[g.tails]))
         assert engine.count_conflicts_dev(dg, torch.from_numpy(colors).cuda()) == exp
+
+
+def test_degree_sums_of_rows_up_to_256():
+    """Weighted degrees of rows of 65 to 256 entries (eight lanes each, 32
+    entries a turn), at and around the turns' ends, with 257 for the next form.
+    Integer weights: the sums are exact and the labels equal the oracle's."""
+    nv, rng = 3000, np.random.default_rng(4)
+    deg = [65, 71, 72, 73, 95, 96, 97, 127, 128, 129, 191, 192, 193, 255, 256, 257, 66]
+    hubs = np.arange(0, 7 * len(deg), 7)
+    rest = np.setdiff1d(np.arange(nv), hubs)
+    pairs = np.concatenate([np.stack([np.full(d, h), rng.choice(rest, d, replace=False)], 1) for h, d in zip(hubs, deg)]
+                           + [np.stack([rest[:-1], rest[1:]], 1)])
+    g = Graph.from_pairs(nv, pairs, rng.integers(1, 8, len(pairs)).astype(np.float64))
+    np.testing.assert_array_equal(g.degrees()[hubs], deg)
+    C, st = engine.runMultiPhaseBasic(g)
+    Co, so = oracle.run_basic(g)
+    np.testing.assert_array_equal(C, Co)
+    assert st["final_modularity"] == so["final_modularity"]
