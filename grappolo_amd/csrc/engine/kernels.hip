@@ -196,14 +196,28 @@ __global__ void k_bin_keys(const i64 *off, i64 nv, const int32_t *colors, int nc
         keys[i] = (uint32_t)(b * ncol + c);
     }
 }
+// start[lo .. hi] = at for every lane's own range; called by whole wavefronts,
+// which fill the longer ranges together (one thread alone took 1.0 ms for the
+// 42,856 keys that a contracted star of 300,001 vertices leaves out).
+constexpr i64 kFillAlone = 16;
+__device__ inline void fill_starts(i64 *start, i64 lo, i64 hi, i64 at) {
+    u64 longer = __ballot(hi - lo >= kFillAlone);
+    if (hi - lo < kFillAlone)
+        for (i64 r = lo; r <= hi; r++) start[r] = at;
+    for (; longer; longer &= longer - 1) {
+        const int src = __ffsll((long long)longer) - 1;
+        const i64 h = __shfl((long long)hi, src), a = __shfl((long long)at, src);
+        for (i64 r = __shfl((long long)lo, src) + threadIdx.x % kWave; r <= h; r += kWave) start[r] = a;
+    }
+}
 // start[k] = first position of key k in the sorted keys (n when absent past the end)
-__global__ void k_slice_starts(const uint32_t *keys, i64 n, i64 nkeys, i64 *start) {
-    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
-        const i64 k = keys[i];
-        const i64 prev = i == 0 ? -1 : (i64)keys[i - 1];
-        for (i64 kk = prev + 1; kk <= k; kk++) start[kk] = i;
-        if (i == n - 1)
-            for (i64 kk = k + 1; kk <= nkeys; kk++) start[kk] = n;
+__global__ __launch_bounds__(kBlock) void k_slice_starts(const uint32_t *keys, i64 n, i64 nkeys, i64 *start) {
+    const int lane = threadIdx.x % kWave;
+    for (i64 i0 = blockIdx.x * (i64)kBlock + threadIdx.x - lane; i0 < n; i0 += (i64)gridDim.x * kBlock) {
+        const i64 i = i0 + lane;
+        const i64 k = i < n ? (i64)keys[i] : -1, prev = i > 0 && i < n ? (i64)keys[i - 1] : -1;
+        fill_starts(start, prev + 1, k, i);
+        fill_starts(start, i == n - 1 ? k + 1 : 0, i == n - 1 ? nkeys : -1, n);
     }
 }
 __global__ void k_perm_degree(const i64 *perm, const i64 *off, i64 n, i64 *degp) {
@@ -3249,17 +3263,22 @@ __global__ __launch_bounds__(kBlock) void k_coarsen_emit(const i64 *off, const i
 // weights (1M-vertex RMAT fold: 15.7M pairs, 1.9 ms of sorting and copying and
 // 0.6 ms of mirroring went; the fold takes 3.4 ms, 5.0 before).  startl[r], startu[r]: pairs before row r's
 // run in either order, so off[r] = startl[r] + startu[r].
-__global__ void k_coarsen_lower(const u64 *ukeys, i64 nu, i64 k, int kb, uint32_t *bkeys, uint32_t *idx,
+__global__ __launch_bounds__(kBlock) void k_coarsen_lower(const u64 *ukeys, i64 nu, i64 k, int kb, uint32_t *bkeys, uint32_t *idx,
                                 i64 *startl) {
     const u64 mask = ((u64)1 << kb) - 1;
-    for (i64 q = blockIdx.x * (i64)blockDim.x + threadIdx.x; q < nu; q += (i64)gridDim.x * blockDim.x) {
-        const u64 key = ukeys[q], a = key >> kb, b = key & mask;
-        bkeys[q] = a != b ? (uint32_t)b : (uint32_t)k;  // a self-loop appears once: its key sorts last
-        idx[q] = (uint32_t)q;
-        const i64 ap = q == 0 ? -1 : (i64)(ukeys[q - 1] >> kb);
-        for (i64 r = ap + 1; r <= (i64)a; r++) startl[r] = q;
-        if (q == nu - 1)
-            for (i64 r = (i64)a + 1; r <= k; r++) startl[r] = nu;
+    const int lane = threadIdx.x % kWave;
+    for (i64 q0 = blockIdx.x * (i64)kBlock + threadIdx.x - lane; q0 < nu; q0 += (i64)gridDim.x * kBlock) {
+        const i64 q = q0 + lane;
+        i64 a = -1, ap = -1;
+        if (q < nu) {
+            const u64 key = ukeys[q], b = key & mask;
+            a = (i64)(key >> kb);
+            if (q > 0) ap = (i64)(ukeys[q - 1] >> kb);
+            bkeys[q] = a != (i64)b ? (uint32_t)b : (uint32_t)k;  // a self-loop appears once: its key sorts last
+            idx[q] = (uint32_t)q;
+        }
+        fill_starts(startl, ap + 1, a, q);
+        fill_starts(startl, q == nu - 1 ? a + 1 : 0, q == nu - 1 ? k : -1, nu);
     }
 }
 __global__ void k_coarsen_rows(const u64 *ukeys, const double *usums, i64 nu, i64 k, int kb, const uint32_t *bkeys,

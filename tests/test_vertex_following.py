@@ -110,3 +110,19 @@ def test_build_vf_with_empty_clusters():
     out = engine.buildNewGraphVF(e, np.array([0, 1, 2], np.int64), 3)
     np.testing.assert_array_equal(out.edgeListPtrs, [0, 0, 0, 0])
     assert out.nnz == 0 and out.numEdges == 0
+
+
+@pytest.mark.parametrize("hubs", [[0], [2999], [0, 15, 31, 48, 65, 129, 194, 800, 2999]])
+def test_contraction_with_runs_of_keys_left_out(hubs):
+    """Rows whose pairs all lie with a few others leave runs of keys out of the
+    sorted pairs (15 to 17, 63 to 65, hundreds, thousands of them, at the start
+    and at the end), which one thread or a wavefront fills: stars around `hubs`
+    contracted with every vertex its own cluster equal the oracle's graphs,
+    seeded and not."""
+    nv = 3000
+    rng = np.random.default_rng(len(hubs))
+    leaves = np.setdiff1d(np.arange(nv), hubs)
+    g = Graph.from_pairs(nv, np.stack([np.array(hubs)[rng.integers(0, len(hubs), len(leaves))], leaves], 1))
+    C = np.arange(nv, dtype=np.int64)
+    _same_graph(engine.buildNextLevelGraphOpt(g, C, nv), oracle.coarsen(g, C, nv))
+    _same_graph(engine.buildNewGraphVF(g, C, nv), oracle.build_vf(g, C, nv))
