@@ -1,8 +1,10 @@
 // Device block cache behind DBuf (declared in common.hpp).
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <string>
 #include <tuple>
 #include <vector>
 
@@ -30,6 +32,16 @@ size_t size_class(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
+// GLV_MAX_BLOCK in the environment: larger requests fail as out of memory (for
+// tests of what a call does then)
+size_t max_block() {
+    static const size_t most = [] {
+        const char *e = std::getenv("GLV_MAX_BLOCK");
+        return e ? (size_t)std::strtoull(e, nullptr, 10) : ~size_t(0);
+    }();
+    return most;
+}
+
 int current_dev() {
     int d = 0;
     (void)hipGetDevice(&d);
@@ -40,6 +52,7 @@ int current_dev() {
 
 void *block_get(size_t bytes, hipStream_t s, size_t *cap) {
     const size_t c = size_class(bytes);
+    if (c > max_block()) fail(GLV_E_OOM, "block of " + std::to_string(c) + " bytes: beyond GLV_MAX_BLOCK");
     const Key k{current_dev(), s, c};
     {
         std::lock_guard<std::mutex> lk(g_blocks_mu);
@@ -109,7 +122,11 @@ unsigned g_stage_gen = 1;
 
 void block_trim() {
     std::lock_guard<std::mutex> lk(g_blocks_mu);
-    trim_locked(current_dev());
+    const int dev = current_dev();
+    trim_locked(dev);
+    // the pool keeps freed memory and serves it to like sizes: back to the device
+    hipMemPool_t pool;
+    if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
 }
 
 void blocks_shutdown() {

@@ -18,6 +18,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include "kernels.hpp"
+#include "wide.hpp"
 #include "mlp_device.hpp"
 #include "sweep_device.hpp"
 
@@ -3165,7 +3166,7 @@ __device__ inline i64 row_index(const ChunkRows &R, const i64 *s_off, const i64 
     return R.r0 + lo;
 }
 __global__ __launch_bounds__(kBlock) void k_entry_labels(const i64 *off, const i64 *tails, const double *w, i64 nv,
-                                                         i64 nnz, int32_t *lab, double *selfw) {
+                                                         i64 nnz, uint32_t *lab, double *selfw) {
     __shared__ i64 s_off[kCoarsenRows + 1], s_r[2];
     const i64 nchunks = (nnz + kCoarsenChunk - 1) / kCoarsenChunk;
     for (i64 ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
@@ -3174,7 +3175,7 @@ __global__ __launch_bounds__(kBlock) void k_entry_labels(const i64 *off, const i
         const i64 r1 = R.r0 + R.nr;
         for (i64 j = e0 + threadIdx.x; j < e1; j += kBlock) {
             const i64 t = tails[j];
-            lab[j] = (int32_t)t;
+            lab[j] = (uint32_t)t;
             // only a neighbour among the chunk's own rows can be the row itself
             if (t >= R.r0 && t < r1 && row_index(R, s_off, off, j) == t) atomicAdd(&selfw[t], w[j]);
         }
@@ -3918,7 +3919,7 @@ void launch_mod_sums(const double *rk, const double *re, const double *a, i64 nv
     k_mod_total<<<1, kSumBlock, 0, s>>>(part, nb, out);
     GLV_LAUNCH_CHECK();
 }
-void launch_entry_labels(const DevGraph &g, int32_t *lab, double *selfw, hipStream_t s) {
+void launch_entry_labels(const DevGraph &g, uint32_t *lab, double *selfw, hipStream_t s) {
     launch_fill_f64(selfw, g.nv, 0.0, s);
     const i64 nch = coarsen_chunks(g.nnz);
     if (nch <= 0) return;
@@ -3926,14 +3927,11 @@ void launch_entry_labels(const DevGraph &g, int32_t *lab, double *selfw, hipStre
                                                                          selfw);
     GLV_LAUNCH_CHECK();
 }
-__global__ void k_positions(const int32_t *tails, i64 n, uint32_t *keys, uint32_t *pos) {
-    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
-        keys[i] = (uint32_t)tails[i];
+__global__ void k_positions(i64 n, uint32_t *pos) {
+    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x)
         pos[i] = (uint32_t)i;
-    }
 }
-void group_entries_by_tail(const DevGraph &g, const int32_t *tails32, DBuf<uint32_t> &pos, i64 *start,
-                           hipStream_t s) {
+void group_entries_by_tail(const DevGraph &g, DBuf<uint32_t> &lab, DBuf<uint32_t> &pos, i64 *start, hipStream_t s) {
     const i64 n = g.nnz;
     pos.alloc(std::max<i64>(n, 1), s);
     if (n <= 0) {
@@ -3942,12 +3940,15 @@ void group_entries_by_tail(const DevGraph &g, const int32_t *tails32, DBuf<uint3
     }
     int bits = 1;
     while (((i64)1 << bits) < g.nv) bits++;
-    DBuf<uint32_t> k0(n, s), k1(n, s), p1(n, s);
-    k_positions<<<grid_for(n, kBlock, 16384), kBlock, 0, s>>>(tails32, n, k0.p, pos.p);
+    {
+        DBuf<uint32_t> k1(n, s), p1(n, s);
+        k_positions<<<grid_for(n, kBlock, 16384), kBlock, 0, s>>>(n, pos.p);
+        GLV_LAUNCH_CHECK();
+        sort_pairs_u32_u32(lab, k1, pos, p1, n, bits, s);
+    }
+    k_slice_starts<<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(lab.p, n, g.nv, start);
     GLV_LAUNCH_CHECK();
-    sort_pairs_u32_u32(k0, k1, pos, p1, n, bits, s);
-    k_slice_starts<<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(k0.p, n, g.nv, start);
-    GLV_LAUNCH_CHECK();
+    launch_narrow_ids(g.tails, n, (int32_t *)lab.p, s);
 }
 // stable; k0, v0: the pairs, then the sorted pairs (k1, v1: n scratch each)
 template <class K, class V>

@@ -101,12 +101,12 @@ void launch_mod_sums(const double *rk, const double *re, const double *a, i64 nv
 
 // --- entry labels (whole-GPU sweep) ----------------------------------------
 // lab[j] = tails[j] as 32 bits; selfw[v] = the weight of v's self-loop entries
-void launch_entry_labels(const DevGraph &g, int32_t *lab, double *selfw, hipStream_t s);
+void launch_entry_labels(const DevGraph &g, uint32_t *lab, double *selfw, hipStream_t s);
 // the entries grouped by neighbour: pos[start[v] .. start[v + 1]) are the
-// positions j with tails[j] == v (g.nnz < 2^32); tails32: the neighbours as
-// launch_entry_labels wrote them
-void group_entries_by_tail(const DevGraph &g, const int32_t *tails32, DBuf<uint32_t> &pos, i64 *start,
-                           hipStream_t s);
+// positions j with tails[j] == v (g.nnz < 2^32); lab: the neighbours as
+// launch_entry_labels wrote them, sorted on the way and written again
+// (16 bytes per entry while it runs, lab and pos among them)
+void group_entries_by_tail(const DevGraph &g, DBuf<uint32_t> &lab, DBuf<uint32_t> &pos, i64 *start, hipStream_t s);
 
 // --- sweeps --------------------------------------------------------------
 // number of block partials the sweep of `bin` writes for `count` vertices

@@ -429,6 +429,104 @@ static i64 mod_part_count(const PhaseSetup &P) {
     return n + kRedBlocks;
 }
 
+// What a colored phase on the whole-GPU sweep holds: the labels as 32 bits (the
+// phase's until its end), the labels per entry, the entry positions grouped by
+// neighbour, the plan and the sweep's state.
+struct WidePhase {
+    WidePlan plan;
+    DBuf<uint32_t> lab, tpos;
+    DBuf<int32_t> c, tgt;
+    DBuf<i64> toff, cperm, cstart, moves;
+    DBuf<double> selfw, re, part, mpart, mout;
+    DBuf<CommInfo> m0, m1;
+    DBuf<unsigned> bar;
+    WideArgs W{};
+};
+
+// Sets X up for a grid of nb workgroups; false when the graph does not suit the
+// sweep's items or its 16 to 20 bytes per entry do not fit the device's memory
+// (the phase then takes the other routes, which need neither).
+bool Engine::setup_wide(const DevGraph &g, const i64 *C, const int32_t *colors, int ncol, const PhaseSetup &P,
+                        int nb, WidePhase &X) {
+    const i64 nv = g.nv;
+    try {
+        X.lab.alloc(std::max<i64>(g.nnz, 1), s_);
+        X.selfw.alloc(nv, s_);
+        launch_entry_labels(g, X.lab.p, X.selfw.p, s_);
+        if (!build_wide_plan(g, P, X.selfw.p, nb, X.plan, s_)) {
+            X = WidePhase();
+            return false;
+        }
+        X.toff.alloc(nv + 1, s_);
+        group_entries_by_tail(g, X.lab, X.tpos, X.toff.p, s_);
+        X.cperm.alloc(nv, s_);
+        X.cstart.alloc(ncol + 1, s_);
+        X.c.alloc(nv, s_);
+        X.tgt.alloc(nv, s_);
+        X.re.alloc(nv, s_);
+        X.m0.alloc(nv, s_);
+        X.m1.alloc(nv, s_);
+        X.part.alloc(2 * (size_t)nb, s_);
+        X.mpart.alloc(3 * kModBlocks, s_);
+        X.mout.alloc(3, s_);
+        X.moves.alloc(1, s_);
+        X.bar.alloc(16 + 16 * (size_t)nb, s_);
+        launch_color_major(P.perm.p, colors, nv, ncol, X.cperm.p, X.cstart.p, s_);
+        launch_narrow_ids(C, nv, X.c.p, s_);
+        launch_fill_i64(X.moves.p, 1, 0, s_);
+    } catch (const Error &e) {
+        if (e.code != GLV_E_OOM) throw;
+        (void)hipGetLastError();
+        X = WidePhase();
+        glv::trace("  wide phase: %s", e.msg.c_str());
+        return false;
+    }
+    const WidePlan &L = X.plan;
+    WideArgs &W = X.W;
+    W.w = g.w;
+    W.k = P.k.p;
+    W.constant = P.constant;
+    W.nv = nv;
+    W.C = X.c.p;
+    W.tgt = X.tgt.p;
+    W.over = L.over.p;
+    W.lab = (int32_t *)X.lab.p;
+    W.tpos = X.tpos.p;
+    W.toff = X.toff.p;
+    W.selfw = X.selfw.p;
+    W.a = P.a.p;
+    W.n = P.n.p;
+    W.m0 = X.m0.p;
+    W.m1 = X.m1.p;
+    W.rows = L.rows.p;
+    W.cperm = X.cperm.p;
+    W.classes = L.classes.p;
+    W.ncls = L.ncls;
+    W.rank = L.rank.p;
+    W.witems = L.witems.p;
+    W.wbeg = L.wbeg.p;
+    W.wend = L.wend.p;
+    W.pitems = L.pitems.p;
+    W.pbeg = L.pbeg.p;
+    W.pend = L.pend.p;
+    W.live = (int)nv;
+    W.giants = L.giants.p;
+    W.ngiants = L.ngiants;
+    W.gpk = L.gpk.p;
+    W.gpv = L.gpv.p;
+    W.gcnt = L.gcnt.p;
+    W.gstate = L.gstate.p;
+    W.gsc = L.gsc.p;
+    W.gcand = L.gcand.p;
+    W.gcid = L.gcid.p;
+    W.gparts = L.gparts;
+    W.gout = L.gout.p;
+    W.bar = X.bar.p;
+    W.part = X.part.p;
+    W.moves = X.moves.p;
+    return true;
+}
+
 // ----------------------------------------------------------- colored phase
 // algoLouvainWithDistOneColoring, Coloring/parallelLouvainWithColoring.cpp:47-286.
 // With a learned active set (las), see LasParams.
@@ -503,6 +601,10 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
             if (tune_.wide_blocks > 0) wblocks = std::min(wblocks, tune_.wide_blocks);
         }
     }
+    if (nv >= (i64(1) << 31) || g.nnz >= (i64(1) << 32)) wblocks = 0;  // 32-bit ids and positions
+    WidePhase X;
+    if (wblocks > 0 && !setup_wide(g, C, colors, ncol, P, wblocks, X)) wblocks = 0;
+    bool use_wide = wblocks > 0;
     // coarse graphs (small, or many small color classes): one persistent
     // launch per iteration (all colors + modularity), grid sized to the color
     // classes: every extra workgroup only lengthens the barriers
@@ -523,7 +625,6 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
             }
         }
     }
-    bool use_wide = wblocks > 0;
     DBuf<i64> gkeys;
     DBuf<double> gvals;
     i64 gslots = 0;
@@ -556,86 +657,18 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     }
     DBuf<unsigned> bar(pblocks > 0 ? kBarrierWords : 0, s_);
     DBuf<double> ppart(pblocks > 0 ? 2 * pblocks : 0, s_);
-    if (use_wide && (nv >= (i64(1) << 31) || g.nnz >= (i64(1) << 32))) use_wide = false;  // 32-bit ids and positions
-    const bool dbl = pblocks > 0 || use_wide;
-    DBuf<i64> cperm(dbl ? nv : 0, s_), cstart(dbl ? ncol + 1 : 0, s_);
+    DBuf<i64> cperm(pblocks > 0 ? nv : 0, s_), cstart(pblocks > 0 ? ncol + 1 : 0, s_);
     // second state buffers of the persistent sweep (one grid barrier per color step)
     DBuf<i64> pC1(pblocks > 0 ? nv : 0, s_), pn1(pblocks > 0 ? nv : 0, s_);
     DBuf<double> pa1(pblocks > 0 ? nv : 0, s_);
     DBuf<uint16_t> pl16(pblocks >= 2 && nv <= kDenseMaxNV ? 2 * nv : 0, s_);  // the dense form's 16-bit labels
-    if (dbl) launch_color_major(P.perm.p, colors, nv, ncol, cperm.p, cstart.p, s_);
+    if (pblocks > 0) launch_color_major(P.perm.p, colors, nv, ncol, cperm.p, cstart.p, s_);
     bool persistent = pblocks > 0;
-    WidePlan WP;
-    WideArgs W{};
-    DBuf<unsigned> wbar(use_wide ? 16 + 16 * (size_t)wblocks : 0, s_);
-    DBuf<double> wpart(use_wide ? 2 * (size_t)wblocks : 0, s_);
-    DBuf<i64> wmoves(use_wide ? 1 : 0, s_);
-    DBuf<CommInfo> wm0(use_wide ? nv : 0, s_), wm1(use_wide ? nv : 0, s_);
-    // the wide sweep's 32-bit labels, the labels held per entry and the entry
-    // positions grouped by neighbour; while it runs, the phase's labels live in
-    // wc (copied back to C at the end of the phase)
-    DBuf<int32_t> wlab(use_wide ? std::max<i64>(g.nnz, 1) : 0, s_);
-    DBuf<double> wself(use_wide ? nv : 0, s_);
-    if (use_wide) {
-        launch_entry_labels(g, wlab.p, wself.p, s_);
-        use_wide = build_wide_plan(g, P, wself.p, wblocks, WP, s_);
-    }
-    DBuf<int32_t> wc(use_wide ? nv : 0, s_), wtgt(use_wide ? nv : 0, s_);
-    DBuf<double> wre(use_wide ? nv : 0, s_), wmpart(use_wide ? 3 * kModBlocks : 0, s_), wmout(use_wide ? 3 : 0, s_);
-    DBuf<uint32_t> wtpos;
-    DBuf<i64> wtoff(use_wide ? nv + 1 : 0, s_);
-    bool labels32 = false;
+    bool labels32 = use_wide;
     // (the launches take a caller's colors as they come: a full modularity pass
     // per iteration costs them less than the movers' sums after every class)
     const bool valid_colors = use_wide ? classes_proper() : proper == Proper::yes;
-    if (use_wide) {
-        launch_narrow_ids(C, nv, wc.p, s_);
-        group_entries_by_tail(g, wlab.p, wtpos, wtoff.p, s_);
-        labels32 = true;
-        launch_fill_i64(wmoves.p, 1, 0, s_);
-        W.w = g.w;
-        W.k = P.k.p;
-        W.constant = P.constant;
-        W.nv = nv;
-        W.C = wc.p;
-        W.tgt = wtgt.p;
-        W.lab = wlab.p;
-        W.tpos = wtpos.p;
-        W.toff = wtoff.p;
-        W.selfw = wself.p;
-        W.defer = !valid_colors;
-        W.a = P.a.p;
-        W.n = P.n.p;
-        W.m0 = wm0.p;
-        W.m1 = wm1.p;
-        W.rows = WP.rows.p;
-        W.cperm = cperm.p;
-        W.classes = WP.classes.p;
-        W.ncls = WP.ncls;
-        W.over = WP.over.p;
-        W.rank = WP.rank.p;
-        W.witems = WP.witems.p;
-        W.wbeg = WP.wbeg.p;
-        W.wend = WP.wend.p;
-        W.pitems = WP.pitems.p;
-        W.pbeg = WP.pbeg.p;
-        W.pend = WP.pend.p;
-        W.live = (int)nv;
-        W.giants = WP.giants.p;
-        W.ngiants = WP.ngiants;
-        W.gpk = WP.gpk.p;
-        W.gpv = WP.gpv.p;
-        W.gcnt = WP.gcnt.p;
-        W.gstate = WP.gstate.p;
-        W.gsc = WP.gsc.p;
-        W.gcand = WP.gcand.p;
-        W.gcid = WP.gcid.p;
-        W.gparts = WP.gparts;
-        W.gout = WP.gout.p;
-        W.bar = wbar.p;
-        W.part = wpart.p;
-        W.moves = wmoves.p;
-    }
+    X.W.defer = !valid_colors;
     glv::trace("colored phase nv %ld, %d colors: %s (%d workgroups)", (long)nv, ncol,
                use_wide ? "wide persistent sweep" : persistent ? "persistent sweep" : "per-color launches",
                use_wide ? wblocks : pblocks);
@@ -742,32 +775,32 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         if (incremental && !prune) launch_fill_f64(dsum.p, 1, 0.0, s_);
         bool done_iter = false;
         if (use_wide) {
-            launch_fill_i32((int32_t *)wbar.p, (i64)wbar.n, 0, s_);
+            launch_fill_i32((int32_t *)X.bar.p, (i64)X.bar.n, 0, s_);
             const int cls = nv > kPersistMaxNV ? K_WIDE : K_PERSIST;
             Profiler::get().begin(cls, s_);
-            use_wide = launch_wide_iteration(W, wblocks, s_);
+            use_wide = launch_wide_iteration(X.W, wblocks, s_);
             Profiler::get().end(cls, 24.0 * g.nnz + 32.0 * nv, s_);
             if (use_wide) {
-                launch_sum_partials(wpart.p, wblocks, res.p, s_);
-                launch_sum_partials(wpart.p + wblocks, wblocks, res.p + 1, s_);
+                launch_sum_partials(X.part.p, wblocks, res.p, s_);
+                launch_sum_partials(X.part.p + wblocks, wblocks, res.p + 1, s_);
                 double h[2];
                 unsigned state[2] = {0, 0};  // abort flag, communities left
                 Readback rb(s_);
                 rb.add(h, res.p, sizeof(h));
-                rb.add(state, wbar.p, sizeof(state));
+                rb.add(state, X.bar.p, sizeof(state));
                 rb.run();
                 const unsigned abort_flag = state[0];
-                W.live = (int)state[1];
+                X.W.live = (int)state[1];
                 if (abort_flag & 2)
                     fail(GLV_E_UNSUPPORTED, "a partition of a giant vertex's communities outgrew the LDS table");
                 if (abort_flag) fail(GLV_E_DEVICE, "grid barrier of the wide sweep timed out");
                 if (numItrs == 1 || !valid_colors) {
                     // a full pass: the first iteration, or classes that may hold an edge
                     Profiler::get().begin(K_MOD, s_);
-                    launch_row_sums(g, wc.p, wlab.p, nullptr, wre.p, s_);
-                    launch_mod_sums(nullptr, wre.p, nullptr, nv, wmpart.p, wmout.p, s_);
+                    launch_row_sums(g, X.c.p, X.W.lab, nullptr, X.re.p, s_);
+                    launch_mod_sums(nullptr, X.re.p, nullptr, nv, X.mpart.p, X.mout.p, s_);
                     Profiler::get().end(K_MOD, 24.0 * g.nnz + 16.0 * nv, s_);
-                    exx = fetch(wmout.p + 1);
+                    exx = fetch(X.mout.p + 1);
                 } else {
                     // moves of one color step are pairwise non-adjacent, so the
                     // internal weight changes by the sum of the movers' 2(e_yt - e_ys)
@@ -778,7 +811,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
                 done_iter = true;
             } else {
                 // launch refused: this phase continues with per-color launches
-                launch_widen_ids(wc.p, nv, C, s_);
+                launch_widen_ids(X.c.p, nv, C, s_);
                 labels32 = false;
             }
         }
@@ -875,8 +908,8 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         if (numItrs >= kMaxPhaseIters) break;
         prevMod = currMod;
     }
-    if (labels32) launch_widen_ids(wc.p, nv, C, s_);
-    if (wmoves.n && nv > kPersistMaxNV) moves_ += fetch(wmoves.p);  // glv_stats::moves: large graphs only
+    if (labels32) launch_widen_ids(X.c.p, nv, C, s_);
+    if (X.moves.n && nv > kPersistMaxNV) moves_ += fetch(X.moves.p);  // glv_stats::moves: large graphs only
     if (mode) sync();
     if (las_off) {
         las->swept_vertices += (i64)numItrs * nonisolated;

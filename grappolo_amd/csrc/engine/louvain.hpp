@@ -101,6 +101,7 @@ struct PhaseSetup {
 };
 
 struct SweepArgs;
+struct WidePhase;
 // the bin-9 (giant vertex) fields of A for color class c of P
 void giant_args(const PhaseSetup &P, int c, SweepArgs &A);
 
@@ -187,6 +188,8 @@ private:
     template <class T>
     T fetch(const T *dptr);
     i64 conflicting_entries(const DevGraph &g, const int32_t *colors);
+    bool setup_wide(const DevGraph &g, const i64 *C, const int32_t *colors, int ncol, const PhaseSetup &P, int nb,
+                    WidePhase &X);
     double colored_modularity(const DevGraph &g, const PhaseSetup &P, const i64 *C,
                               double *part, double *res, double *exx = nullptr);
 };

@@ -247,33 +247,42 @@ bool build_wide_plan(const DevGraph &g, const PhaseSetup &P, const double *selfw
     L.gparts = gparts;
     L.gpairs = gpairs;
     L.gcounts = gcounts;
-    auto upload = [&](auto &buf, const auto &host) {
-        buf.alloc(std::max<size_t>(host.size(), 1), s);
-        if (!host.empty())
-            GLV_HIP(hipMemcpyAsync(buf.p, host.data(), host.size() * sizeof(host[0]), hipMemcpyHostToDevice, s));
-    };
-    upload(L.classes, classes);
-    if (!extra.empty())
-        GLV_HIP(hipMemcpyAsync(L.rows.p + extra0, extra.data(), extra.size() * sizeof(WideRow), hipMemcpyHostToDevice,
-                               s));
-    L.over.alloc(std::max(ncls, 1), s);
-    upload(L.rank, rank);
-    upload(L.witems, wi);
-    upload(L.wbeg, wbeg);
-    upload(L.wend, wend);
-    upload(L.pitems, pi);
-    upload(L.pbeg, pbeg);
-    upload(L.pend, pend);
-    upload(L.giants, giants);
+    // (everything is allocated before the first copy, which reads the host
+    // vectors until the wait below)
+    auto room = [&](auto &buf, size_t n) { buf.alloc(std::max<size_t>(n, 1), s); };
+    room(L.classes, classes.size());
+    room(L.over, ncls);
+    room(L.rank, rank.size());
+    room(L.witems, wi.size());
+    room(L.wbeg, wbeg.size());
+    room(L.wend, wend.size());
+    room(L.pitems, pi.size());
+    room(L.pbeg, pbeg.size());
+    room(L.pend, pend.size());
+    room(L.giants, giants.size());
     const i64 ng = std::max<i64>(L.ngiants, 1);
-    L.gpk.alloc(std::max<i64>(gpairs, 1), s);
-    L.gpv.alloc(std::max<i64>(gpairs, 1), s);
-    L.gcnt.alloc(std::max<i64>(gcounts, 1), s);
-    L.gstate.alloc(3 * ng, s);
-    L.gsc.alloc(ng, s);
-    L.gout.alloc(ng, s);
-    L.gcand.alloc(3 * ng * gparts, s);
-    L.gcid.alloc(ng * gparts, s);
+    room(L.gpk, gpairs);
+    room(L.gpv, gpairs);
+    room(L.gcnt, gcounts);
+    room(L.gstate, 3 * ng);
+    room(L.gsc, ng);
+    room(L.gout, ng);
+    room(L.gcand, 3 * ng * gparts);
+    room(L.gcid, ng * gparts);
+    auto upload = [&](auto *at, const auto &host) {
+        if (!host.empty())
+            GLV_HIP(hipMemcpyAsync(at, host.data(), host.size() * sizeof(host[0]), hipMemcpyHostToDevice, s));
+    };
+    upload(L.rows.p + extra0, extra);
+    upload(L.classes.p, classes);
+    upload(L.rank.p, rank);
+    upload(L.witems.p, wi);
+    upload(L.wbeg.p, wbeg);
+    upload(L.wend.p, wend);
+    upload(L.pitems.p, pi);
+    upload(L.pbeg.p, pbeg);
+    upload(L.pend.p, pend);
+    upload(L.giants.p, giants);
     GLV_HIP(hipStreamSynchronize(s));  // the host vectors are pageable
     trace("  wide plan: %ld workgroup items, %ld wavefront items, %ld giants (%ld pairs, %ld partitions at most), "
           "%.1f ms on the host",

@@ -8,6 +8,8 @@ at least 99.9 % of the moves of an iteration on FP64 weights."""
 import hashlib
 import json
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -17,6 +19,7 @@ import oracle
 pytestmark = pytest.mark.gpu
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "wide_rmat19.json")
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _sha(*arrays):
@@ -236,3 +239,38 @@ def test_degrees_at_the_item_bounds(stage):
         qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
         assert it == ito and q == qo
         np.testing.assert_array_equal(C, Co)
+
+
+_LITTLE_MEMORY = """
+import numpy as np
+import torch
+import oracle
+from grappolo_amd import engine
+from grappolo_amd.graph import gen_planted
+for nv, degree in ((20000, 24), (4096, 128)):
+    g = gen_planted(nv, 4, degree, 0.3, seed=3)
+    colors, mc = oracle.color_greedy(g)
+    C = torch.empty(nv, dtype=torch.int64, device="cuda")
+    q, it = engine.colored_phase_dev(engine.DeviceGraph(g), C, torch.from_numpy(colors).int().cuda(), mc + 1)
+    qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+    assert it == ito and q == qo and np.array_equal(C.cpu().numpy(), Co)
+print("same", flush=True)
+"""
+
+
+@pytest.mark.parametrize("limit,routes", [(None, ["wide persistent sweep", "wide persistent sweep"]),
+                                          (1 << 20, ["per-color launches", "persistent sweep"])])
+def test_phase_without_the_memory_for_the_sweep(limit, routes):
+    """A phase whose entry labels and positions do not fit the device's memory
+    (blocks above `limit` bytes are refused) takes the per-color launches, a
+    dense one the dense sweep, instead of failing: the oracle's labels,
+    iterations and modularity either way.  In a process of its own, which reads
+    the limit."""
+    env = dict(os.environ, GLV_TRACE="1")
+    if limit:
+        env["GLV_MAX_BLOCK"] = str(limit)
+    r = subprocess.run([sys.executable, "-c", _LITTLE_MEMORY], cwd=ROOT, capture_output=True, text=True, timeout=100,
+                       env=env)
+    assert r.returncode == 0 and r.stdout.strip().endswith("same"), r.stderr[-2000:]
+    took = [line.split(": ")[-1].split(" (")[0] for line in r.stderr.splitlines() if "colored phase nv" in line]
+    assert took == routes
