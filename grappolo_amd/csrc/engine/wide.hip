@@ -945,7 +945,7 @@ __global__ void k_wide_rows(const i64 *perm, const i64 *off, const double *k, co
                             WideRow *rows) {
     for (i64 q = lo + blockIdx.x * (i64)blockDim.x + threadIdx.x; q < hi; q += (i64)gridDim.x * blockDim.x) {
         const i64 v = perm[q], b = off[v];
-        rows[q] = WideRow{b, k[v], selfw[v], (int32_t)v, (int32_t)(off[v + 1] - b)};
+        rows[q] = WideRow{b, k[v], selfw[v], (int32_t)v, wide_row_deg(off[v + 1] - b)};
     }
 }
 

@@ -105,6 +105,11 @@ struct WideRow {
     int32_t v;
     int32_t deg;
 };
+// The entries of a row as a WideRow holds them: a row of a multigraph can have
+// 2^31 and more, which is more than the chunks of a giant hold either way.
+constexpr int32_t wide_row_deg(i64 d) { return d < INT32_MAX ? (int32_t)d : INT32_MAX; }
+static_assert(wide_row_deg(i64(1) << 31) > kWMaxChunks * kWChunk && wide_row_deg((i64(1) << 32) - 1) > kWMaxChunks * kWChunk,
+              "a row that no item serves must look like one");
 // A color class: its vertices cperm[lo, hi) and its wavefront items in order
 // -- the vertices of bin 7 with at most kWMidMaxDeg entries (`nextra` rows from
 // `extra0` on, behind the others), the vertices of bins 6, 5, .. 1 (rows
