@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cstring>
+#include <mutex>
 
 #include "active_set.hpp"
 #include "kernels.hpp"
@@ -47,6 +48,19 @@ int bits_for(i64 x) {  // smallest b with 2^b > x
 constexpr int kMaxPhaseIters = 100000;
 
 }  // namespace
+
+// Held from the launch of a kernel with grid barriers until the host has read
+// its results: one such kernel at a time per device.  Its workgroups wait for
+// one another, so every one has to be resident; of two such grids on two
+// streams (threads of a program, each with its own) each could hold CUs that
+// the other's last workgroups need, until the bounded waits give up with an
+// error.  The calling thread waits for each of these kernels anyway.
+static std::unique_lock<std::mutex> grid_turn() {
+    static std::mutex turn[64];
+    int d = 0;
+    GLV_HIP(hipGetDevice(&d));
+    return std::unique_lock<std::mutex>(turn[d & 63]);
+}
 
 template <class T>
 T Engine::fetch(const T *dptr) {
@@ -280,6 +294,7 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
         i64 h[10] = {hc[0], hc[1], 0, 0, 0, 0, 0, 0, 0, 0};
         GLV_HIP(hipMemcpyAsync(ring.p, h, sizeof(h), hipMemcpyHostToDevice, s_));
         launch_fill_i32((int32_t *)bar.p, kJpBarrierWords, 0, s_);
+        const auto turn = grid_turn();
         Profiler::get().begin(K_COLOR, s_);
         const bool ok = pnb > 0 && launch_jp_persistent(g, colors, cnt.p, cur.small, next.small, cur.large,
                                                         next.large, ring.p, bar.p, err.p, colored, prio.p, code.p,
@@ -777,6 +792,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         if (use_wide) {
             launch_fill_i32((int32_t *)X.bar.p, (i64)X.bar.n, 0, s_);
             const int cls = nv > kPersistMaxNV ? K_WIDE : K_PERSIST;
+            auto turn = grid_turn();
             Profiler::get().begin(cls, s_);
             use_wide = launch_wide_iteration(X.W, wblocks, s_);
             Profiler::get().end(cls, 24.0 * g.nnz + 32.0 * nv, s_);
@@ -789,6 +805,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
                 rb.add(h, res.p, sizeof(h));
                 rb.add(state, X.bar.p, sizeof(state));
                 rb.run();
+                turn.unlock();
                 const unsigned abort_flag = state[0];
                 X.W.live = (int)state[1];
                 if (abort_flag & 2)
@@ -818,6 +835,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
         if (done_iter) {
         } else if (persistent) {
             launch_fill_i32((int32_t *)bar.p, kBarrierWords, 0, s_);
+            auto turn = grid_turn();
             Profiler::get().begin(K_PERSIST, s_);
             persistent = launch_colored_iteration(A, plist, pstart, ncol, bar.p, ppart.p, pblocks, s_,
                                                   mode ? stale.p : nullptr, pC1.p, pa1.p, pn1.p,
@@ -832,6 +850,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
                 rb.add(h, res.p, sizeof(h));
                 rb.add(&abort_flag, bar.p, sizeof(unsigned));
                 rb.run();
+                turn.unlock();
                 if (abort_flag) fail(GLV_E_DEVICE, "grid barrier of the persistent sweep timed out");
                 const double c = P.constant;
                 currMod = h[0] * (double)c - h[1] * (double)c * (double)c;

@@ -241,6 +241,40 @@ def test_degrees_at_the_item_bounds(stage):
         np.testing.assert_array_equal(C, Co)
 
 
+def test_two_threads_on_two_streams():
+    """Two threads of a program cluster two graphs at a time, each on a stream of
+    its own: kernels with grid barriers take turns on the device, so both finish
+    with the results that each has alone."""
+    import threading
+    import torch
+    from grappolo_amd import engine
+    from grappolo_amd.graph import gen_lfr
+    dgs = [engine.DeviceGraph(gen_lfr(nv, seed=nv)) for nv in (200003, 150001)]
+    out = [[], []]
+
+    def work(i, runs):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            C = torch.empty(dgs[i].numVertices, dtype=torch.int64, device="cuda")
+            for _ in range(runs):
+                st = engine.run_colored_dev(dgs[i], C)
+                torch.cuda.current_stream().synchronize()
+                out[i].append((st["final_modularity"], st["total_iterations"], C.cpu().numpy()))
+
+    torch.cuda.synchronize()
+    work(0, 1)
+    work(1, 1)
+    threads = [threading.Thread(target=work, args=(i, 4)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for alone, *runs in out:
+        assert len(runs) == 4
+        for r in runs:
+            assert r[:2] == alone[:2]
+            np.testing.assert_array_equal(r[2], alone[2])
+
+
 _LITTLE_MEMORY = """
 import numpy as np
 import torch
