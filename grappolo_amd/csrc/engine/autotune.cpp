@@ -150,14 +150,16 @@ Tuning autotune_launch(Engine &E, const DevGraph &g, const RunParams &p, int rep
     };
     for (int jb : {64, 128, 256}) {
         Tuning c = best;
-        if (jb == c.jp_blocks) continue;
+        if (jb == c.blocks_for(g.nv)) continue;
         c.jp_blocks = jb;
+        c.auto_jp_blocks = false;
         try_color(c);
     }
-    for (i64 cd : {i64(256), i64(1024), i64(4096)}) {
+    for (i64 cd : {kJpCoreDeg, i64(256), i64(1024), i64(4096)}) {
         Tuning c = best;
-        if (cd == c.core_min_deg) continue;
+        if (cd == c.core_degree()) continue;
         c.core_min_deg = cd;
+        c.auto_core_min_deg = false;
         try_color(c);
     }
     if (runs && g.nnz > 0) {

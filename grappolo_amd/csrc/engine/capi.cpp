@@ -1020,11 +1020,16 @@ int glv_autotune_bins_dev(int64_t nv, int64_t nnz, const int64_t *d_offsets, con
     });
 }
 
+static glv_tuning tuning_out(const glv::Tuning &c) {
+    return glv_tuning{c.jp_blocks, c.persist_blocks, c.wide_blocks,
+                      (c.auto_jp_blocks ? GLV_AUTO_JP_BLOCKS : 0) | (c.auto_core_min_deg ? GLV_AUTO_CORE_MIN_DEG : 0),
+                      c.core_min_deg};
+}
+
 int glv_get_tuning(glv_tuning *t) {
     return guarded([&] {
         if (!t) glv::fail(GLV_E_INVALID_ARG, "null tuning");
-        const glv::Tuning &c = glv::current_tuning();
-        *t = glv_tuning{c.jp_blocks, c.persist_blocks, c.wide_blocks, 0, c.core_min_deg};
+        *t = tuning_out(glv::current_tuning());
     });
 }
 
@@ -1036,6 +1041,10 @@ int glv_set_tuning(const glv_tuning *t) {
         c.persist_blocks = t->persist_blocks;
         c.wide_blocks = t->wide_blocks;
         c.core_min_deg = t->core_min_deg;
+        // a value other than the default is meant, whatever the bit beside it says
+        const glv::Tuning d;
+        c.auto_jp_blocks = (t->automatic & GLV_AUTO_JP_BLOCKS) && c.jp_blocks == d.jp_blocks;
+        c.auto_core_min_deg = (t->automatic & GLV_AUTO_CORE_MIN_DEG) && c.core_min_deg == d.core_min_deg;
         if (!glv::valid_tuning(c)) glv::fail(GLV_E_INVALID_ARG, "launch shapes outside the kernels' limits");
         glv::current_tuning() = c;
     });
@@ -1060,12 +1069,10 @@ int glv_autotune_dev(int64_t nv, int64_t nnz, const int64_t *d_offsets, const in
         std::vector<glv::TuneTrial> log;
         const glv::Tuning t = glv::autotune_launch(E, g, p, reps, runs != 0, &log);
         GLV_HIP(hipStreamSynchronize(s));
-        *best = glv_tuning{t.jp_blocks, t.persist_blocks, t.wide_blocks, 0, t.core_min_deg};
+        *best = tuning_out(t);
         const int n = (int)std::min<size_t>(log.size(), (size_t)cap);
         for (int i = 0; i < n; i++) {
-            const glv::Tuning &c = log[i].t;
-            trials[i] = glv_tune_trial{{c.jp_blocks, c.persist_blocks, c.wide_blocks, 0, c.core_min_deg},
-                                       log[i].stage, 0, log[i].ms};
+            trials[i] = glv_tune_trial{tuning_out(log[i].t), log[i].stage, 0, log[i].ms};
         }
         if (ntrials) *ntrials = (int)log.size();
         if (apply) glv::current_tuning() = t;

@@ -51,20 +51,19 @@ constexpr i64 kPersistMaxBlocksHash = 64;
 constexpr i64 kPersistMaxNV = 1 << 18;
 constexpr i64 kPersistMaxPerColor = 256;
 constexpr int kBarrierWords = 16 + 16 * (int)kPersistMaxBlocks;  // abort word + one 64-byte flag line per workgroup
-// The coloring of a graph of more than 16384 vertices takes a core (its
-// highest degrees, coloured by one workgroup) only when the core starts at
-// this degree or above.  A round costs the core's workgroup 3 us and the whole
-// GPU 15 to 20, while rounds of thousands of light vertices are the GPU's:
-// against a line at degree 1024, RMAT with 250,007 vertices takes 4.8 ms
-// instead of 6.9 and LFR with 200,001 2.4 instead of 4.2; a planted graph of
-// 65,536 vertices of degree 16 would take 1.7 ms instead of 0.84 with a line
-// below 24.  From about a million RMAT vertices on the core is full (16,384)
-// above either line.
+// The launch shapes that the coloring takes when they are left to the engine.
+// A graph of more than 16384 vertices has a core (its highest degrees, coloured
+// by one workgroup) only when the core starts at kJpCoreDeg or above.  A round
+// costs the core's workgroup 3 us and the whole GPU 15 to 20, while rounds of
+// thousands of light vertices are the GPU's: against a line at degree 1024, RMAT
+// with 250,007 vertices takes 4.8 ms instead of 6.9 and LFR with 200,001 2.4
+// instead of 4.2; a planted graph of 65,536 vertices of degree 16 would take 1.7
+// ms instead of 0.84 with a line below 24.  From about a million RMAT vertices
+// on the core is full (16,384) above either line.
 constexpr i64 kJpCoreDeg = 64;
-// The tunable launch shapes' defaults, which leave the choice to the engine
-// (a coloring core at kJpCoreDeg, workgroups of the coloring rounds by size).
-constexpr int kJpBlocks = 64;
-constexpr i64 kJpCoreMinDeg = 1024;
+// Workgroups of the persistent rounds: 64 to 128 (RMAT, 4.2M vertices: 25.1 ms
+// with 64, 23.6 with 128, 24.3 with 256; 250,000: 4.78, 4.82, 4.79).
+constexpr int jp_blocks_for(i64 nv) { return nv < 64 * 4096 ? 64 : nv > 128 * 4096 ? 128 : (int)(nv / 4096); }
 // touched communities of one vertex, listed in LDS: at most min(degree, nv)
 constexpr int kDenseListMax = kDenseMaxNV;
 

@@ -189,15 +189,9 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
     const i64 nv = g.nv;
     if (nv == 0) return -1;
     launch_fill_i32(colors, nv, -1, s_);
-    // The shapes left at their defaults follow the graph.  Workgroups of the
-    // persistent rounds: 64 to 128 (RMAT, 4.2M vertices: 25.1 ms with 64, 23.6
-    // with 128, 24.3 with 256; 250,000: 4.78, 4.82, 4.79).  The core's degree:
-    // kJpCoreDeg.
-    const i64 jp_blocks = tune_.jp_blocks != kJpBlocks ? tune_.jp_blocks
-                                                       : std::min<i64>(2 * kJpBlocks, std::max<i64>(kJpBlocks, nv / 4096));
-    const i64 core_deg = tune_.core_min_deg != kJpCoreMinDeg ? tune_.core_min_deg : kJpCoreDeg;
-    const int pnb = (int)std::min<i64>({(i64)jp_persistent_blocks(), jp_blocks,
-                                         std::max<i64>(4, nv / 2048)});
+    const i64 core_deg = tune_.core_degree();
+    const int pnb = (int)std::min<i64>({(i64)jp_persistent_blocks(), (i64)tune_.blocks_for(nv),
+                                        std::max<i64>(4, nv / 2048)});
     DBuf<i64> ring(10, s_);
     DBuf<unsigned> bar(kJpBarrierWords, s_);
     DBuf<int32_t> cnt(nv, s_), dep(nv, s_), err(1, s_), maxc(1, s_);
@@ -390,8 +384,9 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
         launch_color_tail(g, colors, next.small, next.large, next.giant, deeper, cnt.p, base.p, adj.p, err.p, s_);
         Profiler::get().end(K_COLOR_TAIL, 0.0, s_);
     }
-    glv::trace("coloring nv %ld: core %ld (degree >= %ld), %d rounds after it, depth %d, %d rounds, tail %ld",
-               (long)nv, (long)K, K > 0 ? (long)dcore : -1L, prounds, maxd, rounds, (long)deeper);
+    glv::trace("coloring nv %ld: core %ld (degree >= %ld, from %ld), %d workgroups, %d rounds after it, depth %d, "
+               "%d rounds, tail %ld",
+               (long)nv, (long)K, K > 0 ? (long)dcore : -1L, (long)core_deg, pnb, prounds, maxd, rounds, (long)deeper);
     launch_jp_finish(colors, nv, maxc.p, s_);
     const int32_t e = fetch(err.p);
     if (e & 1) fail(GLV_E_TOO_MANY_COLORS, "distance-1 coloring needs more than 4096 colors");

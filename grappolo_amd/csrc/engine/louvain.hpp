@@ -112,12 +112,14 @@ BinConfig &current_bins();
 // None of them changes a result: they choose grids and which vertices the
 // coloring's core pass takes.
 struct Tuning {
-    int jp_blocks = kJpBlocks;         // grid of the persistent coloring rounds (<= kJpPersistMaxBlocks;
-                                       // the default: by the graph's size)
-    i64 core_min_deg = kJpCoreMinDeg;  // a coloring core of a large graph starts at this degree or above
-                                       // (the default: kJpCoreDeg)
-    int persist_blocks = 64;           // grid of the persistent sweep at most (<= kPersistMaxBlocks)
-    int wide_blocks = 0;               // grid of the whole-GPU sweep at most (0: one workgroup per CU)
+    int jp_blocks = 64;       // grid of the persistent coloring rounds (<= kJpPersistMaxBlocks)
+    i64 core_min_deg = 1024;  // a coloring core of a large graph starts at this degree or above
+    int persist_blocks = 64;  // grid of the persistent sweep at most (<= kPersistMaxBlocks)
+    int wide_blocks = 0;      // grid of the whole-GPU sweep at most (0: one workgroup per CU)
+    // the first two are left to the engine, whatever they say (common.hpp)
+    bool auto_jp_blocks = true, auto_core_min_deg = true;
+    int blocks_for(i64 nv) const { return auto_jp_blocks ? jp_blocks_for(nv) : jp_blocks; }
+    i64 core_degree() const { return auto_core_min_deg ? kJpCoreDeg : core_min_deg; }
 };
 Tuning &current_tuning();
 bool valid_tuning(const Tuning &t);

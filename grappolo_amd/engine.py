@@ -30,15 +30,26 @@ class GlvError(RuntimeError):
         self.code = code
 
 
+class Automatic(int):
+    """A launch shape left to the engine; as a number, the value that it has
+    once it is set to a plain one."""
+
+    def __repr__(self):
+        return f"Automatic({int(self)})"
+
+
 class Tuning(ctypes.Structure):
     """glv_tuning: launch shapes of the coloring rounds, the sweeps and the coloring core."""
     _fields_ = [("jp_blocks", ctypes.c_int32), ("persist_blocks", ctypes.c_int32),
-                ("wide_blocks", ctypes.c_int32), ("reserved", ctypes.c_int32),
+                ("wide_blocks", ctypes.c_int32), ("automatic", ctypes.c_int32),
                 ("core_min_deg", ctypes.c_int64)]
+    AUTO_JP_BLOCKS, AUTO_CORE_MIN_DEG = 1, 2
 
     def as_dict(self):
-        return {"jp_blocks": self.jp_blocks, "persist_blocks": self.persist_blocks,
-                "wide_blocks": self.wide_blocks, "core_min_deg": self.core_min_deg}
+        def of(value, bit):
+            return Automatic(value) if self.automatic & bit else value
+        return {"jp_blocks": of(self.jp_blocks, self.AUTO_JP_BLOCKS), "persist_blocks": self.persist_blocks,
+                "wide_blocks": self.wide_blocks, "core_min_deg": of(self.core_min_deg, self.AUTO_CORE_MIN_DEG)}
 
 
 class TuneTrial(ctypes.Structure):
@@ -639,8 +650,12 @@ def get_tuning():
     return t.as_dict()
 
 
-def set_tuning(jp_blocks=64, persist_blocks=64, wide_blocks=0, core_min_deg=1024):
-    t = Tuning(int(jp_blocks), int(persist_blocks), int(wide_blocks), 0, int(core_min_deg))
+def set_tuning(jp_blocks=Automatic(64), persist_blocks=64, wide_blocks=0, core_min_deg=Automatic(1024)):
+    """Launch shapes of later calls; the values are taken as they stand, the two
+    Automatic ones (left out, or as get_tuning hands them out) by the engine."""
+    auto = ((Tuning.AUTO_JP_BLOCKS if isinstance(jp_blocks, Automatic) else 0)
+            | (Tuning.AUTO_CORE_MIN_DEG if isinstance(core_min_deg, Automatic) else 0))
+    t = Tuning(int(jp_blocks), int(persist_blocks), int(wide_blocks), auto, int(core_min_deg))
     _call("glv_set_tuning", ctypes.byref(t))
 
 

@@ -356,12 +356,16 @@ int glv_autotune_bins_dev(int64_t nv, int64_t nnz, const int64_t *d_offsets, con
  * shapes, keeping a change that saves at least 2 %, and writes the fastest
  * to *best (made current when apply != 0).  trials (cap entries, may be
  * null) receive every measured candidate; *ntrials their count. */
+/* Every value is taken as it stands, unless a bit of `automatic` leaves it to
+ * the engine and it holds the default. */
+#define GLV_AUTO_JP_BLOCKS 1    /* 64 to 128 workgroups by the graph's size */
+#define GLV_AUTO_CORE_MIN_DEG 2 /* the engine's line (degree 64) */
 typedef struct {
-    int32_t jp_blocks;      /* 1..256; 64, the default: 64 to 128 by the graph's size */
+    int32_t jp_blocks;      /* 1..256, default 64 and automatic */
     int32_t persist_blocks; /* 1..256, default 64 (graphs above 15360 vertices: at most 64 used) */
     int32_t wide_blocks;    /* 0: up to one workgroup per CU by the color classes (default), else at most that many */
-    int32_t reserved;
-    int64_t core_min_deg;   /* >= 1; 1024, the default: the engine's line (degree 64) */
+    int32_t automatic;      /* GLV_AUTO_*, default both */
+    int64_t core_min_deg;   /* >= 1, default 1024 and automatic */
 } glv_tuning;
 typedef struct {
     glv_tuning t;

@@ -8,6 +8,9 @@ coloring) and the oracle's coloring."""
 import hashlib
 import json
 import os
+import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -15,6 +18,7 @@ import pytest
 import oracle
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "wide_rmat19.json")
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 DEFAULT = {"jp_blocks": 64, "persist_blocks": 64, "wide_blocks": 0, "core_min_deg": 1024}
 
 
@@ -43,6 +47,66 @@ def test_tuning_limits_and_round_trip():
         assert engine.get_tuning()["persist_blocks"] == 256
     finally:
         engine.set_tuning(**DEFAULT)
+
+
+def test_values_left_to_the_engine():
+    """A fresh process leaves two shapes to the engine; their numbers set as
+    plain ones are meant (also when they equal the defaults), what get_tuning
+    hands out restores the state, and a C caller's change beside a set bit is
+    taken."""
+    code = """
+import ctypes
+from grappolo_amd import engine
+from grappolo_amd.engine import Automatic, Tuning
+def auto():
+    t = engine.get_tuning()
+    return [k for k in t if isinstance(t[k], Automatic)]
+both = ["jp_blocks", "core_min_deg"]
+assert auto() == both
+first = engine.get_tuning()
+engine.set_tuning(jp_blocks=64, core_min_deg=1024)
+assert auto() == [] and engine.get_tuning() == first
+engine.set_tuning(**first)
+assert auto() == both
+engine.set_tuning(core_min_deg=64, wide_blocks=8)
+assert auto() == ["jp_blocks"] and engine.get_tuning()["core_min_deg"] == 64
+engine.set_tuning()
+assert auto() == both
+t = Tuning()
+engine._call("glv_get_tuning", ctypes.byref(t))
+t.core_min_deg = 256
+engine._call("glv_set_tuning", ctypes.byref(t))
+assert auto() == ["jp_blocks"] and engine.get_tuning()["core_min_deg"] == 256
+old = Tuning(64, 64, 0, 0, 1024)  # as saved before there was anything automatic
+engine._call("glv_set_tuning", ctypes.byref(old))
+assert auto() == []
+"""
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=100)
+
+
+@pytest.mark.gpu
+def test_plain_values_are_what_runs():
+    """The coloring takes the workgroups and the core's degree that were set,
+    the numbers of the defaults among them, and the engine's own otherwise; the
+    colors are the same.  In a process of its own, for its trace."""
+    code = """
+import sys
+import numpy as np
+from grappolo_amd import engine
+from grappolo_amd.graph import gen_planted
+g = gen_planted(400000, 100, 6, 0.3, seed=1)
+ref = None
+for kw in ({}, {"jp_blocks": 64}, {"core_min_deg": 1024}, {"jp_blocks": 128, "core_min_deg": 64}, {"core_min_deg": 8}):
+    engine.set_tuning(**kw)
+    colors, mc = engine.algoDistanceOneVertexColoringOpt(g)
+    ref = colors if ref is None else ref
+    assert np.array_equal(colors, ref)
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100,
+                       env=dict(os.environ, GLV_TRACE="1"))
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = re.findall(r"coloring nv 400000: core .*?, from (\d+)\), (\d+) workgroups", r.stderr)
+    assert [(int(d), int(b)) for d, b in got] == [(64, 97), (64, 64), (1024, 97), (64, 128), (8, 97)]
 
 
 @pytest.fixture(scope="module")
