@@ -241,8 +241,9 @@ __global__ void k_mask_graphs(const i64 *vb, i64 ng, const uint8_t *keep, i64 *C
 
 // err |= 1 when an entry of graph g's rows points outside [vb[g], vb[g+1]); a
 // graph's entries are shared by gridDim.y workgroups (one each left the
-// largest of 128 graphs, 1.6M entries, 2.0 ms in a single workgroup)
-constexpr int kCheckSplit = 32;
+// largest of 128 graphs, 1.6M entries, 2.0 ms in a single workgroup), fewer the
+// more graphs there are: a grid of about kCheckGrid
+constexpr i64 kCheckSplit = 32, kCheckGrid = 4096;
 __global__ void k_check_blocks(const i64 *off, const i64 *tails, const i64 *vb, i64 ng, int32_t *err) {
     const i64 step = (i64)gridDim.y * blockDim.x;
     for (i64 g = blockIdx.x; g < ng; g += gridDim.x) {
@@ -262,7 +263,8 @@ __global__ void k_check_blocks(const i64 *off, const i64 *tails, const i64 *vb, 
 
 void launch_check_blocks(const i64 *off, const i64 *tails, const i64 *vb, i64 ng, int32_t *err, hipStream_t s) {
     if (ng <= 0) return;
-    k_check_blocks<<<dim3((unsigned)std::max<i64>(1, std::min<i64>(ng, 65535)), kCheckSplit), kBB, 0, s>>>(off, tails, vb, ng, err);
+    const unsigned split = (unsigned)std::max<i64>(1, std::min(kCheckSplit, kCheckGrid / ng));
+    k_check_blocks<<<dim3((unsigned)std::min<i64>(ng, 65535), split), kBB, 0, s>>>(off, tails, vb, ng, err);
     GLV_LAUNCH_CHECK();
 }
 

@@ -109,6 +109,25 @@ def test_batch_rejects_cross_graph_entries():
         engine.run_basic_batch_dev(dg, np.array([0, 200, 300], np.int64), C)
 
 
+@pytest.mark.parametrize("ng", [2, 128, 129, 4096, 4097])
+def test_one_cross_graph_entry_is_found(ng):
+    """A graph's entries are checked by 32 workgroups or, from 129 graphs on, by
+    fewer, by one from 2049: the one edge that joins two graphs is found, the
+    same graphs without it are taken."""
+    import torch
+    from grappolo_amd import engine
+    from grappolo_amd.graph import Graph
+    at = np.arange(ng)[:, None] * 5
+    paths = np.concatenate([np.stack([at + i, at + i + 1], 2).reshape(-1, 2) for i in range(4)])
+    vb = np.arange(ng + 1, dtype=np.int64) * 5
+    C = torch.empty(5 * ng, dtype=torch.int64, device="cuda")
+    engine.run_basic_batch_dev(engine.DeviceGraph(Graph.from_pairs(5 * ng, paths)), vb, C)
+    for i in (1, ng - 1):
+        joined = Graph.from_pairs(5 * ng, np.concatenate([paths, [[5 * i - 1, 5 * i]]]))
+        with pytest.raises(engine.GlvError):
+            engine.run_basic_batch_dev(engine.DeviceGraph(joined), vb, C)
+
+
 def test_autotuned_bins_keep_results():
     """Bin ranges change only which kernel serves a vertex: with the tuned
     ranges a unit-weight run is identical to the default one."""
