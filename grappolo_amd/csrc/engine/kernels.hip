@@ -3927,24 +3927,46 @@ void launch_entry_labels(const DevGraph &g, uint32_t *lab, double *selfw, hipStr
                                                                          selfw);
     GLV_LAUNCH_CHECK();
 }
-__global__ void k_positions(i64 n, uint32_t *pos) {
-    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x)
-        pos[i] = (uint32_t)i;
+template <class T>
+__global__ void k_positions(i64 n, T *pos) {
+    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) pos[i] = (T)i;
 }
-void group_entries_by_tail(const DevGraph &g, DBuf<uint32_t> &lab, DBuf<uint32_t> &pos, i64 *start, hipStream_t s) {
+__global__ void k_split_positions(const u64 *pos, i64 n, uint32_t *lo, uint8_t *hi) {
+    for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
+        lo[i] = (uint32_t)(pos[i] & ((u64(1) << kTposBits) - 1));
+        hi[i] = (uint8_t)(pos[i] >> kTposBits);
+    }
+}
+// stable; k0, v0: the pairs, then the sorted pairs (k1, v1: n scratch each)
+template <class K, class V>
+static void sort_pairs_buffered(DBuf<K> &k0, DBuf<K> &k1, DBuf<V> &v0, DBuf<V> &v1, i64 n, int end_bit,
+                                hipStream_t s);
+void group_entries_by_tail(const DevGraph &g, DBuf<uint32_t> &lab, DBuf<uint32_t> &pos, DBuf<uint8_t> &hi, i64 *start,
+                           hipStream_t s) {
     const i64 n = g.nnz;
-    pos.alloc(std::max<i64>(n, 1), s);
     if (n <= 0) {
         launch_fill_i64(start, g.nv + 1, 0, s);
         return;
     }
     int bits = 1;
     while (((i64)1 << bits) < g.nv) bits++;
-    {
-        DBuf<uint32_t> k1(n, s), p1(n, s);
-        k_positions<<<grid_for(n, kBlock, 16384), kBlock, 0, s>>>(n, pos.p);
+    auto sorted = [&](auto &p0) {
+        DBuf<uint32_t> k1(n, s);
+        std::remove_reference_t<decltype(p0)> p1(n, s);
+        p0.alloc(n, s);
+        k_positions<<<grid_for(n, kBlock, 16384), kBlock, 0, s>>>(n, p0.p);
         GLV_LAUNCH_CHECK();
-        sort_pairs_u32_u32(lab, k1, pos, p1, n, bits, s);
+        sort_pairs_buffered(lab, k1, p0, p1, n, bits, s);
+    };
+    if (n <= i64(1) << kTposBits) {
+        sorted(pos);
+    } else {
+        DBuf<u64> p;
+        sorted(p);
+        pos.alloc(n, s);
+        hi.alloc(n, s);
+        k_split_positions<<<grid_for(n, kBlock, 16384), kBlock, 0, s>>>(p.p, n, pos.p, hi.p);
+        GLV_LAUNCH_CHECK();
     }
     k_slice_starts<<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(lab.p, n, g.nv, start);
     GLV_LAUNCH_CHECK();

@@ -103,10 +103,13 @@ void launch_mod_sums(const double *rk, const double *re, const double *a, i64 nv
 // lab[j] = tails[j] as 32 bits; selfw[v] = the weight of v's self-loop entries
 void launch_entry_labels(const DevGraph &g, uint32_t *lab, double *selfw, hipStream_t s);
 // the entries grouped by neighbour: pos[start[v] .. start[v + 1]) are the
-// positions j with tails[j] == v (g.nnz < 2^32); lab: the neighbours as
-// launch_entry_labels wrote them, sorted on the way and written again
-// (16 bytes per entry while it runs, lab and pos among them)
-void group_entries_by_tail(const DevGraph &g, DBuf<uint32_t> &lab, DBuf<uint32_t> &pos, i64 *start, hipStream_t s);
+// positions j with tails[j] == v, their low kTposBits bits, the rest in hi
+// (allocated where positions go beyond); lab: the neighbours as
+// launch_entry_labels wrote them, sorted on the way and written again (16 bytes
+// per entry while it runs, 24 with hi, lab and pos among them)
+constexpr int kTposBits = 32;
+void group_entries_by_tail(const DevGraph &g, DBuf<uint32_t> &lab, DBuf<uint32_t> &pos, DBuf<uint8_t> &hi, i64 *start,
+                           hipStream_t s);
 
 // --- sweeps --------------------------------------------------------------
 // number of block partials the sweep of `bin` writes for `count` vertices

@@ -445,6 +445,7 @@ static i64 mod_part_count(const PhaseSetup &P) {
 struct WidePhase {
     WidePlan plan;
     DBuf<uint32_t> lab, tpos;
+    DBuf<uint8_t> tpos_hi;
     DBuf<int32_t> c, tgt;
     DBuf<i64> toff, cperm, cstart, moves;
     DBuf<double> selfw, re, part, mpart, mout;
@@ -454,7 +455,7 @@ struct WidePhase {
 };
 
 // Sets X up for a grid of nb workgroups; false when the graph does not suit the
-// sweep's items or its 16 to 20 bytes per entry do not fit the device's memory
+// sweep's items or its 16 bytes per entry do not fit the device's memory
 // (the phase then takes the other routes, which need neither).
 bool Engine::setup_wide(const DevGraph &g, const i64 *C, const int32_t *colors, int ncol, const PhaseSetup &P,
                         int nb, WidePhase &X) {
@@ -468,7 +469,7 @@ bool Engine::setup_wide(const DevGraph &g, const i64 *C, const int32_t *colors, 
             return false;
         }
         X.toff.alloc(nv + 1, s_);
-        group_entries_by_tail(g, X.lab, X.tpos, X.toff.p, s_);
+        group_entries_by_tail(g, X.lab, X.tpos, X.tpos_hi, X.toff.p, s_);
         X.cperm.alloc(nv, s_);
         X.cstart.alloc(ncol + 1, s_);
         X.c.alloc(nv, s_);
@@ -502,6 +503,7 @@ bool Engine::setup_wide(const DevGraph &g, const i64 *C, const int32_t *colors, 
     W.over = L.over.p;
     W.lab = (int32_t *)X.lab.p;
     W.tpos = X.tpos.p;
+    W.tpos_hi = X.tpos_hi.p;
     W.toff = X.toff.p;
     W.selfw = X.selfw.p;
     W.a = P.a.p;
@@ -611,7 +613,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
             if (tune_.wide_blocks > 0) wblocks = std::min(wblocks, tune_.wide_blocks);
         }
     }
-    if (nv >= (i64(1) << 31) || g.nnz >= (i64(1) << 32)) wblocks = 0;  // 32-bit ids and positions
+    if (nv >= (i64(1) << 31) || g.nnz > kWideMaxEntries) wblocks = 0;  // 32-bit ids
     WidePhase X;
     if (wblocks > 0 && !setup_wide(g, C, colors, ncol, P, wblocks, X)) wblocks = 0;
     bool use_wide = wblocks > 0;

@@ -290,7 +290,11 @@ __device__ inline int32_t decide(const WideArgs &W, const Step &S, Moves &M, int
 // no item of this step reads them; with a coloring whose classes hold edges
 // (W.defer) the labels are written after the step instead.
 __device__ inline void push_label(const WideArgs &W, int32_t v, int32_t t, int first, int step) {
-    for (i64 q = W.toff[v] + first, e = W.toff[v + 1]; q < e; q += step) W.lab[W.tpos[q]] = t;
+    for (i64 q = W.toff[v] + first, e = W.toff[v + 1]; q < e; q += step) {
+        i64 at = W.tpos[q];
+        if (W.tpos_hi) at |= (i64)W.tpos_hi[q] << kTposBits;
+        W.lab[at] = t;
+    }
 }
 
 // Empties the first T slots of an LDS table (the caller synchronises).  Every

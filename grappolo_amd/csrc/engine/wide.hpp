@@ -33,8 +33,8 @@
 // Entries of a class's rows hold labels of other classes, so a move may be
 // written in its own step; with a coloring whose classes hold edges it is
 // written after the step, behind a second barrier (WideArgs::defer).  Entry
-// positions are 32-bit: the sweep serves graphs below 2^32 entries and 2^31
-// vertices.
+// positions are 32-bit words, with a byte more each from 2^32 entries on: the
+// sweep serves graphs below 2^40 entries and 2^31 vertices.
 //
 // Workgroup items are dealt out when the phase starts (longest first, each to
 // the least loaded workgroup), wavefront items in turn to the wavefronts of
@@ -51,6 +51,7 @@
 namespace glv {
 
 constexpr int kWBlock = 1024;            // threads per workgroup
+constexpr i64 kWideMaxEntries = i64(1) << (kTposBits + 8);  // entry positions of a word and a byte
 constexpr int kWHeavySlots = 12288;      // LDS table of a workgroup: u32 keys + f64 values
 constexpr i64 kWHeavyMaxDeg = 8192;      // larger vertices are giants (several workgroups)
 constexpr i64 kWChunk = 4096;            // entries of a giant per accumulation item
@@ -152,6 +153,7 @@ struct WideArgs {
     int32_t *over;               // per class: such a move was made
     int32_t *lab;                // per adjacency entry, the label of its neighbour
     const uint32_t *tpos;        // the entries whose neighbour is v: tpos[toff[v]] .. tpos[toff[v + 1]]
+    const uint8_t *tpos_hi;      // their bits from kTposBits on; null when there are none
     const i64 *toff;
     const double *selfw;         // self-loop weight of every vertex
     bool defer;                  // a class may hold an edge: labels enter `lab` after the step

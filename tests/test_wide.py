@@ -308,3 +308,44 @@ def test_phase_without_the_memory_for_the_sweep(limit, routes):
     assert r.returncode == 0 and r.stdout.strip().endswith("same"), r.stderr[-2000:]
     took = [line.split(": ")[-1].split(" (")[0] for line in r.stderr.splitlines() if "colored phase nv" in line]
     assert took == routes
+
+
+_MANY_ENTRIES = """
+import hashlib
+import torch
+from grappolo_amd import engine
+n, k = 256 * 34000, 255  # vertex v beside v - k .. v + k, colors v mod (k + 1)
+step = torch.cat([torch.arange(-k, 0, device="cuda"), torch.arange(1, k + 1, device="cuda")])
+tails = torch.empty(n * 2 * k, dtype=torch.int64, device="cuda")
+assert tails.shape[0] > 1 << 32
+for r in range(0, n, 1 << 18):
+    rows = torch.arange(r, min(n, r + (1 << 18)), device="cuda")
+    tails[r * 2 * k:(r + rows.shape[0]) * 2 * k] = ((rows[:, None] + step) % n).reshape(-1)
+w = torch.ones(tails.shape[0], dtype=torch.float64, device="cuda")
+dg = engine.DeviceGraph.from_tensors(torch.arange(n + 1, device="cuda") * (2 * k), tails, w, n * k)
+torch.cuda.empty_cache()
+colors = (torch.arange(n, device="cuda") % (k + 1)).int()
+C = torch.empty(n, dtype=torch.int64, device="cuda")
+print("built", flush=True)
+q, it = engine.colored_phase_dev(dg, C, colors, k + 1, -1.0, 1e-2)
+print(repr(q), it, hashlib.sha256(C.cpu().numpy().tobytes()).hexdigest(), flush=True)
+"""
+
+
+def test_more_entries_than_a_word_counts():
+    """4.4 billion entries: positions beyond 32 bits take a byte more, and a
+    phase of the whole-GPU sweep gives the labels and modularity of the
+    per-color launches (unit weights).  In processes of their own, one after the
+    other; needs about 180 GB of device memory."""
+    import torch
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 220 << 30:
+        pytest.skip("device memory")
+    res = []
+    for wide in ("1", "0"):
+        r = subprocess.run([sys.executable, "-c", _MANY_ENTRIES], cwd=ROOT, capture_output=True, text=True, timeout=110,
+                           env=dict(os.environ, GLV_TRACE="1", GLV_WIDE=wide))
+        assert r.returncode == 0, r.stderr[-2000:]
+        assert ("wide persistent sweep" in r.stderr) == (wide == "1")
+        res.append(r.stdout.splitlines()[-1])
+    assert res[0] == res[1]
