@@ -71,9 +71,10 @@ def pendants(seed=17, nv=5000, weighted=True):
 def cliques(seed=13, nv=20000, size=200, inter=8, hub_degrees=(5000, 4500), weighted=False):
     """Dense near-cliques (every coloring needs ~size colors, so classes hold
     ~nv/size vertices) joined by random inter-clique edges, plus hubs: a graph
-    above the dense-accumulator limit that the persistent sweep serves with its
-    LDS hash (and, past kPHashMaxDeg, the dense view in slabs or, above two
-    slabs of vertices, the HBM table)."""
+    above the dense-accumulator limit that the persistent sweep, where it takes
+    the place of the whole-GPU one (pruned and trace runs, GLV_WIDE=0), serves
+    with its LDS hash (and, past kPHashMaxDeg, the dense view in slabs or, above
+    two slabs of vertices, the HBM table)."""
     rng = np.random.default_rng(seed)
     blocks = nv // size
     pairs = []

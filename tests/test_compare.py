@@ -101,8 +101,9 @@ def test_gini_equals_oracle(n):
 @pytest.mark.parametrize("nc", [1, 2, 1023, 16384, 16385, 40000])
 def test_sizes_on_both_sides_of_the_lds_limit(nc):
     """Community sizes are counted in LDS up to 16,384 communities and with
-    device atomics above: counts and Gini coefficients equal the oracle's, and
-    a label past the last community is still refused."""
+    device atomics above: counts and Gini coefficients equal the oracle's.  A
+    label below -1 is refused (none lies past the last community: the largest
+    one makes their number)."""
     rng = np.random.default_rng(nc)
     n = 50021
     a, b = rng.integers(0, nc, n), rng.integers(0, max(nc // 2, 1), n)
@@ -111,3 +112,6 @@ def test_sizes_on_both_sides_of_the_lds_limit(nc):
     exp, _, _ = oracle.compare(a, b)
     got, _, _ = engine.computeCommunityComparisons(a, b)
     _same(got, exp)
+    for bad in ((np.where(np.arange(n) == 77, -2, a), b), (a, np.where(np.arange(n) == n - 1, -2, b))):
+        with pytest.raises(engine.GlvError):
+            engine.computeCommunityComparisons(*bad)

@@ -184,11 +184,11 @@ def test_plain_phase(name, nomap):
 @pytest.mark.parametrize("nv,size", [(20000, 200), (40000, 300)])
 @pytest.mark.parametrize("weighted", [False, True])
 def test_colored_phase_persistent_hash(weighted, nv, size):
-    """Graphs above the dense-accumulator limit with small color classes: the
-    persistent sweep with per-workgroup LDS hash tables, and for the two hubs
-    the dense LDS view one slab of communities at a time (20,000 vertices: two
-    slabs) or the HBM table (40,000 vertices), against the oracle's frozen
-    color steps."""
+    """Graphs above the dense-accumulator limit with small color classes and two
+    hubs, against the oracle's frozen color steps: the whole-GPU sweep here; the
+    persistent sweep with LDS hash tables that pruned runs take, and the
+    launches per color, on the same graphs in
+    test_routes_without_the_whole_gpu_sweep."""
     from graphs import cliques
     g = cliques(weighted=weighted, nv=nv, size=size)
     colors, mc = oracle.color_greedy(g)
@@ -514,3 +514,49 @@ def test_degree_sums_of_rows_up_to_256():
     Co, so = oracle.run_basic(g)
     np.testing.assert_array_equal(C, Co)
     assert st["final_modularity"] == so["final_modularity"]
+
+
+_WITHOUT_WIDE = """
+import sys
+sys.path.insert(0, "tests")
+import numpy as np
+import oracle
+from grappolo_amd import engine
+from graphs import catalog, cliques, unit_weights
+graphs = {f"cliques {w} {nv}": cliques(weighted=w, nv=nv, size=size)
+          for w in (False, True) for nv, size in ((20000, 200), (40000, 300))}
+graphs.update({k: v for k, v in catalog().items() if k in ("lfr_w", "hubs_big", "hubs_giant")})
+for name, g in graphs.items():
+    colors, mc = oracle.color_greedy(g)
+    print("graph", name, file=sys.stderr, flush=True)
+    q, C, it = engine.algoLouvainWithDistOneColoring(g, colors, mc + 1, -1.0, 1e-6)
+    qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+    if unit_weights(g):
+        assert it == ito and q == qo and np.array_equal(C, Co), name
+    else:
+        assert abs(q - qo) < 1e-3, (name, q, qo)
+print("equal", flush=True)
+"""
+
+
+def test_routes_without_the_whole_gpu_sweep():
+    """GLV_WIDE=0 (read once per process): small classes take the persistent
+    sweep with per-workgroup LDS hash tables, its hubs the dense LDS view one
+    slab of communities at a time (20,000 vertices: two slabs) or the HBM table
+    (40,000), and graphs with large classes the launches per color, hubs of more
+    than 2,048 and 16,384 entries among them.  The oracle's frozen color steps."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _WITHOUT_WIDE], cwd=root, capture_output=True, text=True, timeout=110,
+                       env=dict(os.environ, GLV_TRACE="1", GLV_WIDE="0"))
+    assert r.returncode == 0 and r.stdout.strip().endswith("equal"), r.stderr[-2000:]
+    took, at = {}, None
+    for line in r.stderr.splitlines():
+        if line.startswith("graph "):
+            at = line[6:]
+        elif "colored phase nv" in line:
+            took[at] = line.split(": ")[-1].split(" (")[0]
+    hashed = {f"cliques {w} {nv}": "persistent sweep" for w in (False, True) for nv in (20000, 40000)}
+    assert took == {**hashed, **dict.fromkeys(("lfr_w", "hubs_big", "hubs_giant"), "per-color launches")}

@@ -1,10 +1,11 @@
 """The whole-GPU persistent colored iteration (engine/wide.hip): graphs above
-262,144 vertices sweep every color step of an iteration in one launch, with
-light, mid, heavy and giant vertices as work items of wavefronts and
-workgroups.  Checked against the oracle's restatement of the colored sweep
-(Coloring/parallelLouvainWithColoring.cpp:154-218) and multi-phase driver
-(Coloring/runMultiPhaseColoring.cpp:51-238): bit-identical on unit weights,
-at least 99.9 % of the moves of an iteration on FP64 weights."""
+15,360 vertices, and smaller ones with large color classes, sweep every color
+step of an iteration in one launch, with light, mid, heavy and giant vertices as
+work items of wavefronts and workgroups.  Phases of few, light and large classes
+take launches per color instead.  Checked against the oracle's restatement of
+the colored sweep (Coloring/parallelLouvainWithColoring.cpp:154-218) and
+multi-phase driver (Coloring/runMultiPhaseColoring.cpp:51-238): bit-identical
+on unit weights, at least 99.9 % of the moves of an iteration on FP64 weights."""
 import hashlib
 import json
 import os
