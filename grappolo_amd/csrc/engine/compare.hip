@@ -97,10 +97,11 @@ __global__ void k_sizes(const i64 *C, i64 n, i64 base, i64 nc, unsigned long lon
     }
 }
 
-// The same through counts in LDS, for at most kLdsSizes communities: device
-// atomics run at about 3.5e9/s whatever the address, so one per vertex took 605
-// us for 2,000,003 labels of 4000 communities; here a workgroup adds its
-// communities once (26 us).  The grid keeps those additions near 2^17.
+// The same through counts in LDS, for at most kLdsSizes communities: a device
+// atomic per vertex took 605 us for 2,000,003 labels of 4000 communities
+// (3.3e9/s; on ten communities they queue, 14.6 ms the whole comparison); here a
+// workgroup adds its communities once (26 us, 0.3 ms).  The grid keeps those
+// additions near 2^17.
 constexpr i64 kLdsSizes = 16384;
 constexpr int kSizesBlock = 1024;
 __global__ __launch_bounds__(kSizesBlock) void k_sizes_lds(const i64 *C, i64 n, i64 base, int nc,

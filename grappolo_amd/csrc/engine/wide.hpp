@@ -3,11 +3,11 @@
 //
 // One launch per colored iteration (all color steps of the iteration, the
 // per-color loop of Coloring/parallelLouvainWithColoring.cpp:169-218 with the
-// community updates of :213-217) on a grid of one 1024-thread workgroup per
-// CU, with one grid barrier per color step.  The work of a color step is a
-// list of items fixed when the phase starts:
-//   workgroup items: a heavy vertex (257..kWHeavyMaxDeg entries, LDS table of
-//     the whole workgroup), a chunk of kWChunk entries of a giant vertex
+// community updates of :213-217) on a grid of 1024-thread workgroups, at most
+// one per CU (wide_grid), with one grid barrier per color step.  The work of a
+// color step is a list of items fixed when the phase starts:
+//   workgroup items: a heavy vertex (kWMidMaxDeg + 1..kWHeavyMaxDeg entries, LDS
+//     table of the whole workgroup), a chunk of kWChunk entries of a giant vertex
 //     (summed per community in LDS, then written out as (community, weight)
 //     pairs grouped by a hash partition of the community ids) and a
 //     partition of a giant's communities (its pairs from every chunk summed in
@@ -79,8 +79,11 @@ constexpr i64 kWideDensePerColor = 64;
 constexpr i64 kWideLightNV = 524288, kWideLightEntries = 250000;
 constexpr double kWideLightLaunches = 2.2;
 
-// Relative costs of workgroup items (microseconds, measured order of
-// magnitude): a heavy vertex kWCostHeavy plus three per 1024 entries.
+// Relative costs of workgroup items (about microseconds): a heavy vertex
+// kWCostHeavy plus three per 1024 entries.  Runs hardly depend on them (RMAT of
+// 4.2M vertices, RMAT of 250,007, LFR of 1M, ms: 1420, 110.4, 48.8; workgroup
+// items at half 1441, 110.5, 48.9; one per 1024 entries 1420, 110.7, 48.9;
+// wavefront items at half 1428, 110.8, 48.9, at 1.7 times 1425, 110.3, 48.7).
 constexpr double kWCostHeavy = 10.0, kWCostChunk = 10.0, kWCostPart = 10.0;
 // wavefront items: a mid vertex, a batch of light vertices (a workgroup runs
 // kWWavesPerGroup of them at a time)
