@@ -176,7 +176,7 @@ void run_basic_batch(Engine &E, const DevGraph &g0, const std::vector<i64> &vb0,
                     launch_sweep(b, true, A, s);
                 }
                 launch_isolated_targets(P.perm.p + P.bin_lo(0), P.bin_hi(0) - P.bin_lo(0), tgt, s);
-                launch_graph_mod(d_vb.p, ng, d_active.p, eii.p, P.a.p, d_exx.p, d_a2.p, s, d_done.p);
+                launch_graph_mod(d_vb.p, ng, nv, d_active.p, eii.p, P.a.p, d_exx.p, d_a2.p, s, d_done.p);
                 launch_batch_decide(d_vb.p, ng, d_exx.p, d_a2.p, d_gconst.p, d_lower.p, p.threshold, kMaxPhaseIters,
                                     d_prev.p, d_curr.p, d_itrs.p, d_active.p, d_apply.p, d_done.p, d_live.p, s);
                 launch_batch_apply(nv, gid.p, d_apply.p, tgt, curr, past, P.k.p, P.a.p, P.n.p, s, d_done.p);

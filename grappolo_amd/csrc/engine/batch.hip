@@ -42,21 +42,25 @@ __global__ __launch_bounds__(kBB) void k_graph_const(const i64 *vb, i64 ng, cons
     }
 }
 
-// per active graph: internal weight and sum of squared community degrees
-// (a workgroup per graph: the largest graphs, 50,000 vertices, set its time --
-// 19 us with 256 threads and one load in flight, 7 us with 1024 and two)
+// per active graph: internal weight and sum of squared community degrees, a
+// workgroup of B threads per graph.  The largest graphs, 50,000 vertices, set its
+// time in a batch of the usual sizes (19 us with 256 threads and one load in
+// flight, 7 us with 1024 and two); thousands of small ones fill the GPU by
+// themselves and take kBB (a batch of 4096 graphs of 20 vertices 4.9 ms with 1024
+// threads, 4.3 so).
 constexpr int kGraphModBlock = 1024;
-__global__ __launch_bounds__(kGraphModBlock) void k_graph_mod(const i64 *vb, i64 ng, const uint8_t *active,
-                                                              const double *eii, const double *a, double *exx,
-                                                              double *a2, const int32_t *skip) {
-    __shared__ double sh[2][kGraphModBlock / kWave];
+constexpr i64 kGraphModMean = 1024;  // vertices per graph on average from which on
+template <int B>
+__global__ __launch_bounds__(B) void k_graph_mod(const i64 *vb, i64 ng, const uint8_t *active, const double *eii,
+                                                 const double *a, double *exx, double *a2, const int32_t *skip) {
+    __shared__ double sh[2][B / kWave];
     if (skip && *skip) return;
     for (i64 g = blockIdx.x; g < ng; g += gridDim.x) {
         if (!active[g]) continue;
         const i64 end = vb[g + 1];
         double e = 0, q = 0;
-        for (i64 v = vb[g] + threadIdx.x; v < end; v += 2 * kGraphModBlock) {
-            const i64 u = v + kGraphModBlock;
+        for (i64 v = vb[g] + threadIdx.x; v < end; v += 2 * B) {
+            const i64 u = v + B;
             const double ev = eii[v], av = a[v], eu = u < end ? eii[u] : 0.0, au = u < end ? a[u] : 0.0;
             e += ev + eu;
             q += av * av + au * au;
@@ -74,7 +78,7 @@ __global__ __launch_bounds__(kGraphModBlock) void k_graph_mod(const i64 *vb, i64
         __syncthreads();
         if (threadIdx.x == 0) {
             e = q = 0;
-            for (int x = 0; x < kGraphModBlock / kWave; x++) {
+            for (int x = 0; x < B / kWave; x++) {
                 e += sh[0][x];
                 q += sh[1][x];
             }
@@ -291,10 +295,13 @@ void launch_graph_const(const i64 *vb, i64 ng, const double *k, double *gconst, 
     k_graph_const<<<graph_grid(ng), kBB, 0, s>>>(vb, ng, k, gconst);
     GLV_LAUNCH_CHECK();
 }
-void launch_graph_mod(const i64 *vb, i64 ng, const uint8_t *active, const double *eii, const double *a,
+void launch_graph_mod(const i64 *vb, i64 ng, i64 nv, const uint8_t *active, const double *eii, const double *a,
                       double *exx, double *a2, hipStream_t s, const int32_t *skip) {
     if (ng <= 0) return;
-    k_graph_mod<<<graph_grid(ng), kGraphModBlock, 0, s>>>(vb, ng, active, eii, a, exx, a2, skip);
+    if (nv / ng >= kGraphModMean)
+        k_graph_mod<kGraphModBlock><<<graph_grid(ng), kGraphModBlock, 0, s>>>(vb, ng, active, eii, a, exx, a2, skip);
+    else
+        k_graph_mod<kBB><<<graph_grid(ng), kBB, 0, s>>>(vb, ng, active, eii, a, exx, a2, skip);
     GLV_LAUNCH_CHECK();
 }
 void launch_batch_decide(const i64 *vb, i64 ng, const double *exx, const double *a2, const double *gconst,

@@ -37,7 +37,7 @@ void run_basic_batch(Engine &E, const DevGraph &g0, const std::vector<i64> &vb0,
 void launch_fill_gid(const i64 *vb, i64 ng, int32_t *gid, hipStream_t s);
 void launch_graph_const(const i64 *vb, i64 ng, const double *k, double *gconst, hipStream_t s);
 // skip: nothing to do when *skip is set (after every graph's phase has ended)
-void launch_graph_mod(const i64 *vb, i64 ng, const uint8_t *active, const double *eii, const double *a,
+void launch_graph_mod(const i64 *vb, i64 ng, i64 nv, const uint8_t *active, const double *eii, const double *a,
                       double *exx, double *a2, hipStream_t s, const int32_t *skip = nullptr);
 void launch_batch_decide(const i64 *vb, i64 ng, const double *exx, const double *a2, const double *gconst,
                          const double *lower, double thresh, int maxitr, double *prev, double *curr, int32_t *itrs,
