@@ -7,8 +7,8 @@
 #include <atomic>
 #include <chrono>
 #include <new>
-#include <thread>
 
+#include "host_workers.hpp"
 #include "louvain.hpp"
 #include "wide.hpp"
 
@@ -175,10 +175,7 @@ bool build_wide_plan(const DevGraph &g, const PhaseSetup &P, const double *selfw
             }
         }
     };
-    std::vector<std::thread> pool;
-    for (int t = 1; t < nthreads; t++) pool.emplace_back(worker);
-    worker();
-    for (auto &t : pool) t.join();
+    run_workers(nthreads, worker);
     if (no_memory) throw std::bad_alloc();
     // the non-empty classes, and every workgroup's streams over them
     std::vector<WideClass> classes;

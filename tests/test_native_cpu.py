@@ -197,3 +197,42 @@ def test_read_communities_keeps_the_reference_parse(tmp_path):
         p = tmp_path / f"c{i}"
         p.write_bytes(text)
         np.testing.assert_array_equal(driver.read_communities(p), np.array(exp, np.int64))
+
+
+_WORKERS = r"""
+#include <sys/resource.h>
+#include <atomic>
+#include <cstdio>
+#include "host_workers.hpp"
+int main(int, char **) {
+    for (int tight = 0; tight < 2; tight++) {
+        if (tight) {  // no room for a thread's stack
+            std::FILE *f = std::fopen("/proc/self/statm", "r");
+            long pages = 0;
+            if (!f || std::fscanf(f, "%ld", &pages) != 1) return 2;
+            std::fclose(f);
+            struct rlimit r{(rlim_t)pages * 4096 + (1 << 20), RLIM_INFINITY};
+            if (setrlimit(RLIMIT_AS, &r)) return 3;
+        }
+        std::atomic<int> next{0}, done{0};
+        glv::run_workers(16, [&] {
+            while (next++ < 1000) done++;
+        });
+        if (done != 1000) return 4;
+    }
+    std::puts("done");
+}
+"""
+
+
+def test_workers_without_threads_to_be_had(tmp_path):
+    """Host work shared by threads is done by those the system gives, here by
+    the calling one alone, instead of ending the program."""
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src = tmp_path / "workers.cpp"
+    src.write_text(_WORKERS)
+    subprocess.run(["g++", "-std=c++17", "-pthread", "-I", os.path.join(root, "grappolo_amd", "csrc", "engine"), str(src),
+                    "-o", str(tmp_path / "workers")], check=True, timeout=100)
+    r = subprocess.run([str(tmp_path / "workers")], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "done", (r.returncode, r.stderr)
