@@ -434,10 +434,12 @@ def main():
     tuning = None
     if not args.no_autotune:
         t = time.perf_counter()
+        def shapes(sh):  # with the names of those left to the engine
+            return {**sh, "automatic": [k for k in sh if isinstance(sh[k], engine.Automatic)]}
         default = engine.get_tuning()
         best, log = engine.autotune_dev(dg, runs=True, apply=True, reps=1, **params)
-        tuning = {"default": default, "chosen": best, "seconds": round(time.perf_counter() - t, 1),
-                  "trials": [{"shapes": sh, "timed_on": stage, "ms": round(ms, 2)} for sh, stage, ms in log]}
+        tuning = {"default": shapes(default), "chosen": shapes(best), "seconds": round(time.perf_counter() - t, 1),
+                  "trials": [{"shapes": shapes(sh), "timed_on": stage, "ms": round(ms, 2)} for sh, stage, ms in log]}
         print(f"[bench] autotune: {best} in {tuning['seconds']} s", file=sys.stderr, flush=True)
 
     for i in range(args.warmup):
