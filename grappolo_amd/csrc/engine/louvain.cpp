@@ -580,17 +580,22 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     // iteration, most of it one HBM-table launch per class), a 62,103-vertex
     // coarse phase of 69 colors from 45.2 to 14.9 ms.
     //
-    // Not so where the launches are few and full (wide.hpp, kWideLight*): no
+    // Not so where the launches are few and full (wide.hpp, kWideLight): no
     // vertex above 256 entries, and a class takes about two launches or is
     // large.  They need no item plan and no entry positions, and a class takes
     // them 10 us against a color step's 13.  Per-color launches / this sweep, ms
-    // per phase: path of 200,000 0.4 / 0.9, grid of 400 x 400 1.4 / 2.4, of 700 x
-    // 700 2.1 / 3.4, planted 65,536 of degree 128 2.5 / 3.6, 200,000 of 128 4.8 /
-    // 6.3 and of 40 8.3 / 9.7, 500,000 of 32 14.0 / 17.1, 260,000 of 24 in 17
-    // classes 14.3 / 16.3.  On the other side: planted 65,536 of degree 16
-    // (105,000 entries and 3.1 launches a class) 5.4 / 4.9, 20,000 of degree 8 2.6
-    // / 2.1; a million of degree 100 26.3 / 21.7 (the gathered labels outgrow an
-    // XCD's L2).
+    // per phase of a caller's colors: path of 200,000 0.4 / 0.9, grid of 400 x 400
+    // 1.4 / 2.4, of 700 x 700 2.1 / 3.4, planted 65,536 of degree 128 2.5 / 3.6,
+    // 200,000 of 128 4.8 / 6.3 and of 40 8.3 / 9.7, 500,000 of 32 14.0 / 17.1,
+    // 260,000 of 24 in 17 classes 14.3 / 16.3.  On the other side: planted 65,536
+    // of degree 16 (105,000 entries and 3.1 launches a class) 5.4 / 4.9, 20,000 of
+    // degree 8 2.6 / 2.1; a million of degree 100 26.3 / 21.7 (the gathered labels
+    // outgrow an XCD's L2).  A run's fresh coloring is known to be proper: the
+    // sweep need not find that out, and the launches add up the movers' weights,
+    // so the line lies higher: planted 65,536 of degree 64 (190,000 entries and
+    // 1.7 launches a class) 8.7 / 7.6 and 6.1 / 5.9, 200,000 of 16 (320,000, 3.4)
+    // 19.5 / 17.9 and 10.4 / 10.2, but 200,000 of 40 (500,000, 2.1) 8.8 / 9.9,
+    // 260,000 of 24 (480,000, 2.8) 9.5 / 10.3.
     //
     // Dense phases (<= 15,360 vertices) with classes of kWideDensePerColor
     // vertices or more take it too (the dense sweep gives every vertex a
@@ -603,9 +608,10 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     const bool las_mode = las && !(las->mode == 2 && nv <= kDenseMaxNV) && las->mode != 0;
     int wblocks = 0;
     if (!las_mode && nonempty > 0 && nv / nonempty <= kWideMaxPerColor && wide_enabled()) {
+        const WideLight line = proper == Proper::yes ? kWideLightRun : kWideLight;
         const bool light = P.bin_hi(kNumBins - 1) == P.bin_lo(7) && per_class > kPersistMaxPerColor &&
                            nv <= kWideLightNV &&
-                           (bins <= kWideLightLaunches * nonempty || g.nnz / nonempty >= kWideLightEntries);
+                           (bins <= line.launches * nonempty || g.nnz / nonempty >= line.entries);
         if (nv > kDenseMaxNV ? !light
                              : per_class >= kWideDensePerColor &&
                                    (per_class >= 2 * kWideDensePerColor || classes_proper())) {

@@ -74,10 +74,15 @@ constexpr i64 kWideDensePerColor = 64;
 
 // Phases without a vertex above 256 entries keep the per-color launches up to
 // kWideLightNV vertices (64-bit labels within an XCD's 4 MB L2) when a class
-// takes kWideLightLaunches of them on average or holds kWideLightEntries entries
+// takes at most `launches` of them on average or holds `entries` entries
 // (measured where the choice is made, Engine::colored_phase).
-constexpr i64 kWideLightNV = 524288, kWideLightEntries = 250000;
-constexpr double kWideLightLaunches = 2.2;
+struct WideLight {
+    double launches;
+    i64 entries;
+};
+constexpr WideLight kWideLight{2.2, 250000};     // a caller's colors, classes that hold edges
+constexpr WideLight kWideLightRun{1.5, 400000};  // a coloring known to be proper
+constexpr i64 kWideLightNV = 524288;
 
 // Relative costs of workgroup items (about microseconds): a heavy vertex
 // kWCostHeavy plus three per 1024 entries.  Runs hardly depend on them (RMAT of

@@ -311,6 +311,34 @@ def test_phase_without_the_memory_for_the_sweep(limit, routes):
     assert took == routes
 
 
+_RUN_AND_STAGE = """
+import numpy as np
+import oracle
+from grappolo_amd import engine
+from grappolo_amd.graph import gen_planted
+g = gen_planted(20000, 16, 60, 0.25, seed=2)  # bins of 33 to 64 and 65 to 256 entries
+C, st = engine.runMultiPhaseColoring(g, minGraphSize=20001)
+Co, so = oracle.run_colored(g, coloring="jp", frozen=True, minGraphSize=20001)
+assert st["final_modularity"] == so["final_modularity"] and np.array_equal(C, Co)
+colors, mc, _ = oracle.color_jp(g)
+q, C, it = engine.algoLouvainWithDistOneColoring(g, colors.astype(np.int32), mc + 1, -1.0, 1e-6)
+qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
+assert it == ito and q == qo and np.array_equal(C, Co)
+print("same", flush=True)
+"""
+
+
+def test_route_of_a_run_and_of_a_callers_colors():
+    """Classes of two launches each: a run, whose coloring is known to be
+    proper, takes the whole-GPU sweep, the stage call with the same colors the
+    launches; both equal the oracle."""
+    r = subprocess.run([sys.executable, "-c", _RUN_AND_STAGE], cwd=ROOT, capture_output=True, text=True, timeout=100,
+                       env=dict(os.environ, GLV_TRACE="1"))
+    assert r.returncode == 0 and r.stdout.strip().endswith("same"), r.stderr[-2000:]
+    took = [line.split(": ")[-1].split(" (")[0] for line in r.stderr.splitlines() if "colored phase nv 20000" in line]
+    assert took == ["wide persistent sweep", "per-color launches"]
+
+
 _MANY_ENTRIES = """
 import hashlib
 import torch
