@@ -3768,17 +3768,17 @@ void launch_jp_finish(int32_t *state, i64 nv, int32_t *maxc, hipStream_t s) {
     GLV_LAUNCH_CHECK();
 }
 void launch_color_conflicts(const DevGraph &g, const int32_t *colors, i64 *count, hipStream_t s) {
+    launch_fill_i64(count, 2, 0, s);
     if (g.nv <= 0) return;
     DBuf<i64> hubs(g.nv, s);
-    DBuf<unsigned long long> nhubs(1, s);
-    launch_fill_i64((i64 *)nhubs.p, 1, 0, s);
+    unsigned long long *nhubs = (unsigned long long *)count + 1;
     with_row_lanes(g, [&](auto lanes) {
         constexpr int G = decltype(lanes)::value;
         k_color_conflicts<G><<<grid_for(g.nv * G, kBlock, 8192), kBlock, 0, s>>>(g.off, g.tails, g.nv, colors, count,
-                                                                                 hubs.p, nhubs.p);
+                                                                                 hubs.p, nhubs);
     });
     GLV_LAUNCH_CHECK();
-    k_color_conflicts_hub<<<256, kSumBlock, 0, s>>>(g.off, g.tails, colors, count, hubs.p, nhubs.p);
+    k_color_conflicts_hub<<<256, kSumBlock, 0, s>>>(g.off, g.tails, colors, count, hubs.p, nhubs);
     GLV_LAUNCH_CHECK();
 }
 

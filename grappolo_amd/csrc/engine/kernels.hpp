@@ -269,6 +269,7 @@ constexpr int kJpDepthWindow = 4096;
 void launch_jp_depth_hist(const int32_t *dep, i64 nv, int32_t top, unsigned *hist, hipStream_t s);
 // vertices deeper than rounds become uncoloured (the tail)
 void launch_jp_depth_cut(const int32_t *dep, i64 nv, int32_t rounds, int32_t *colors, hipStream_t s);
+// count[0] = entries whose ends share a color, self-loops aside (count[1]: scratch)
 void launch_color_conflicts(const DevGraph &g, const int32_t *colors, i64 *count, hipStream_t s);
 
 // --- renumber / compose --------------------------------------------------

@@ -397,8 +397,7 @@ int Engine::color(const DevGraph &g, int32_t *colors, int *rounds_out) {
 }
 
 i64 Engine::conflicting_entries(const DevGraph &g, const int32_t *colors) {
-    DBuf<i64> c(1, s_);
-    launch_fill_i64(c.p, 1, 0, s_);
+    DBuf<i64> c(2, s_);
     launch_color_conflicts(g, colors, c.p, s_);
     return fetch(c.p);
 }
@@ -594,8 +593,9 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     // sweep need not find that out, and the launches add up the movers' weights,
     // so the line lies higher: planted 65,536 of degree 64 (190,000 entries and
     // 1.7 launches a class) 8.7 / 7.6 and 6.1 / 5.9, 200,000 of 16 (320,000, 3.4)
-    // 19.5 / 17.9 and 10.4 / 10.2, but 200,000 of 40 (500,000, 2.1) 8.8 / 9.9,
-    // 260,000 of 24 (480,000, 2.8) 9.5 / 10.3.
+    // 19.5 / 17.9 and 10.4 / 10.2, a ring of 40,000 of degree 200 (283 vertices a
+    // class, one launch) 98 / 82 the whole run, but 200,000 of 40 (500,000, 2.1)
+    // 8.8 / 9.9, 260,000 of 24 (480,000, 2.8) 9.5 / 10.3.
     //
     // Dense phases (<= 15,360 vertices) with classes of kWideDensePerColor
     // vertices or more take it too (the dense sweep gives every vertex a
@@ -609,8 +609,7 @@ double Engine::colored_phase(const DevGraph &g, i64 *C, const int32_t *colors, i
     int wblocks = 0;
     if (!las_mode && nonempty > 0 && nv / nonempty <= kWideMaxPerColor && wide_enabled()) {
         const WideLight line = proper == Proper::yes ? kWideLightRun : kWideLight;
-        const bool light = P.bin_hi(kNumBins - 1) == P.bin_lo(7) && per_class > kPersistMaxPerColor &&
-                           nv <= kWideLightNV &&
+        const bool light = P.bin_hi(kNumBins - 1) == P.bin_lo(7) && per_class > line.vertices && nv <= kWideLightNV &&
                            (bins <= line.launches * nonempty || g.nnz / nonempty >= line.entries);
         if (nv > kDenseMaxNV ? !light
                              : per_class >= kWideDensePerColor &&

@@ -74,14 +74,15 @@ constexpr i64 kWideDensePerColor = 64;
 
 // Phases without a vertex above 256 entries keep the per-color launches up to
 // kWideLightNV vertices (64-bit labels within an XCD's 4 MB L2) when a class
-// takes at most `launches` of them on average or holds `entries` entries
-// (measured where the choice is made, Engine::colored_phase).
+// holds more than `vertices` on average and takes at most `launches` of them or
+// holds `entries` entries (measured where the choice is made,
+// Engine::colored_phase).
 struct WideLight {
     double launches;
-    i64 entries;
+    i64 entries, vertices;
 };
-constexpr WideLight kWideLight{2.2, 250000};     // a caller's colors, classes that hold edges
-constexpr WideLight kWideLightRun{1.5, 400000};  // a coloring known to be proper
+constexpr WideLight kWideLight{2.2, 250000, kPersistMaxPerColor};  // a caller's colors, classes that hold edges
+constexpr WideLight kWideLightRun{1.5, 400000, 1024};              // a coloring known to be proper
 constexpr i64 kWideLightNV = 524288;
 
 // Relative costs of workgroup items (about microseconds): a heavy vertex

@@ -312,31 +312,41 @@ def test_phase_without_the_memory_for_the_sweep(limit, routes):
 
 
 _RUN_AND_STAGE = """
+import sys
 import numpy as np
 import oracle
 from grappolo_amd import engine
-from grappolo_amd.graph import gen_planted
-g = gen_planted(20000, 16, 60, 0.25, seed=2)  # bins of 33 to 64 and 65 to 256 entries
-C, st = engine.runMultiPhaseColoring(g, minGraphSize=20001)
-Co, so = oracle.run_colored(g, coloring="jp", frozen=True, minGraphSize=20001)
+from grappolo_amd.graph import Graph, gen_planted
+nv = int(sys.argv[1])
+if nv < 50000:
+    g = gen_planted(nv, 16, 60, 0.25, seed=2)  # bins of 33 to 64 and 65 to 256 entries
+else:
+    i = np.arange(nv)
+    g = Graph.from_pairs(nv, np.concatenate([np.stack([i, (i + s) % nv], 1) for s in range(1, 21)]))
+C, st = engine.runMultiPhaseColoring(g, minGraphSize=nv + 1)
+Co, so = oracle.run_colored(g, coloring="jp", frozen=True, minGraphSize=nv + 1)
 assert st["final_modularity"] == so["final_modularity"] and np.array_equal(C, Co)
 colors, mc, _ = oracle.color_jp(g)
 q, C, it = engine.algoLouvainWithDistOneColoring(g, colors.astype(np.int32), mc + 1, -1.0, 1e-6)
 qo, Co, ito, _ = oracle.louvain_colored(g, colors, mc + 1, -1.0, 1e-6, frozen=True)
 assert it == ito and q == qo and np.array_equal(C, Co)
-print("same", flush=True)
+print("same", nv / (mc + 1), flush=True)
 """
 
 
-def test_route_of_a_run_and_of_a_callers_colors():
-    """Classes of two launches each: a run, whose coloring is known to be
-    proper, takes the whole-GPU sweep, the stage call with the same colors the
-    launches; both equal the oracle."""
-    r = subprocess.run([sys.executable, "-c", _RUN_AND_STAGE], cwd=ROOT, capture_output=True, text=True, timeout=100,
-                       env=dict(os.environ, GLV_TRACE="1"))
-    assert r.returncode == 0 and r.stdout.strip().endswith("same"), r.stderr[-2000:]
-    took = [line.split(": ")[-1].split(" (")[0] for line in r.stderr.splitlines() if "colored phase nv 20000" in line]
-    assert took == ["wide persistent sweep", "per-color launches"]
+@pytest.mark.parametrize("nv,run", [(20000, "wide persistent sweep"), (30000, "wide persistent sweep"),
+                                    (50000, "per-color launches")])
+def test_route_of_a_run_and_of_a_callers_colors(nv, run):
+    """A run's coloring is known to be proper: classes of up to 1,024 vertices, or
+    of more than one and a half launches each, take the whole-GPU sweep there,
+    where the stage call with the same colors takes the launches (952 and 1,400
+    vertices a class, 1.7 launches; 1,500 and one launch: both take them).  All
+    equal the oracle."""
+    r = subprocess.run([sys.executable, "-c", _RUN_AND_STAGE, str(nv)], cwd=ROOT, capture_output=True, text=True,
+                       timeout=100, env=dict(os.environ, GLV_TRACE="1"))
+    assert r.returncode == 0 and r.stdout.startswith("same"), r.stderr[-2000:]
+    took = [line.split(": ")[-1].split(" (")[0] for line in r.stderr.splitlines() if f"colored phase nv {nv}" in line]
+    assert took == [run, "per-color launches"]
 
 
 _MANY_ENTRIES = """
